@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
 #include <mutex>
 #include <new>
 #include <string>
@@ -44,9 +45,9 @@ std::vector<fdtd2d::Event> build_events(const fdtd2d_problem *p, std::vector<int
     fdtd2d::Event e;
   };
   std::vector<E> v;
-  for (int e = 0; e < p->nsrc; ++e) v.push_back({p->src_j[e], {p->src_i[e], fdtd2d::EV_SRC, e, 0}});
-  for (int d = 0; d < p->ndet; ++d) v.push_back({p->det_j[d], {p->det_i[d], fdtd2d::EV_DET, d, 0}});
-  for (int c = 0; c < p->ncomp; ++c) v.push_back({p->comp_j[c], {p->comp_i[c], fdtd2d::EV_COMP, c, 0}});
+  for (int e = 0; e < p->nsrc; ++e) v.push_back({p->src_j[e], {p->src_i[e], fdtd2d::EV_SRC, e, p->src_j[e]}});
+  for (int d = 0; d < p->ndet; ++d) v.push_back({p->det_j[d], {p->det_i[d], fdtd2d::EV_DET, d, p->det_j[d]}});
+  for (int c = 0; c < p->ncomp; ++c) v.push_back({p->comp_j[c], {p->comp_i[c], fdtd2d::EV_COMP, c, p->comp_j[c]}});
   std::stable_sort(v.begin(), v.end(), [](const E &a, const E &b) {
     if (a.j != b.j) return a.j < b.j;
     if (a.e.kind != b.e.kind) return a.e.kind < b.e.kind;
@@ -430,6 +431,105 @@ Tiling make_tiling(int nx, int ny, int P, int T, int C, int band, int band_cpml,
   return t;
 }
 
+bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMasks *m,
+                 std::vector<fdtd2d::BlockTile> &out) {
+  if (std::min(s.R, s.RG) * s.W <= 2 * T) return false;  // no row left to store
+  const int Pe = std::max(P, 1);
+  auto count = [](const int *pref, int a, int b) { return pref && b > a ? pref[b] - pref[a] : 0; };
+  auto span_hits = [](const int *lo, const int *hi, int r, int c0, int c1) {
+    return lo[r] <= hi[r] && lo[r] < c1 && hi[r] >= c0;
+  };
+  // events of rows [j0, j1), columns [c0, c1)
+  auto events = [&](int j0, int j1, int c0, int c1) {
+    if (!m) return 0;
+    int n = 0;
+    const int2 *e = std::lower_bound(m->ev, m->ev + m->nev, j0, [](const int2 &u, int j) { return u.y < j; });
+    for (; e < m->ev + m->nev && e->y < j1; ++e) n += e->x >= c0 && e->x < c1;
+    return n;
+  };
+  // rows [j0, j1) clear of the y strips, the ring and rows whose den differ
+  auto plain_rows = [&](int j0, int j1) { return j0 > Pe && j1 < ny - Pe - 1 && !(m && count(m->srow_pref, j0, j1)); };
+  out.clear();
+  std::vector<fdtd2d::BlockTile> inner;
+  // the flags of a tile of R rows per wave whose window starts at (c0, w0);
+  // false if a wave holds too many events
+  auto describe = [&](fdtd2d::BlockTile &t, int R, int c1, bool probes) {
+    for (int w = 0; w < s.W; ++w) {
+      // the wave's rows, and the row above them, whose Hx it steps too
+      const int rb = t.rs + w * R, j0 = std::min(rb, ny), je = std::min(rb + R, ny);
+      const int n = events(j0, je, t.cs, c1);
+      if (n > 64) return false;
+      const bool ev = n > 0 || (probes && j0 < je) || (m && count(m->lrow_pref, j0, je));
+      bool jz = !(m && m->ne_lo), full = m && m->ne_run_off && j0 < je;
+      for (int r = j0; r < je; ++r) {
+        if (!jz) jz = span_hits(m->ne_lo, m->ne_hi, r, t.cs, c1) || span_hits(m->jz_lo, m->jz_hi, r, t.cs, c1);
+        if (!full) continue;
+        bool in = false;
+        for (int q = m->ne_run_off[r]; q < m->ne_run_off[r + 1] && !in; ++q)
+          in = m->ne_runs[q].x <= t.cs && m->ne_runs[q].y >= c1;
+        full = in;
+      }
+      t.y_waves |= !plain_rows(rb - 1, rb + R) << w;
+      t.e_waves |= ev << w;
+      t.jz_waves |= jz << w;
+      t.full_waves |= (jz && full) << w;
+    }
+    return true;
+  };
+  // Column pieces: 64*C wide windows where they are clear of the x strips, 64
+  // wide ones at the edges; T columns (rounded up to C) recomputed on each
+  // side that is not the grid's edge.
+  const int halo = (T + s.C - 1) / s.C * s.C, full_w = 64 * s.C;
+  auto plain_cols = [&](int c0, int c1) { return c0 > Pe && c1 < nx - Pe - 1 && !(m && count(m->scol_pref, c0, c1)); };
+  // general tiles over rows [j0, j1) (whose neighbours the windows may reach) of columns [o, oe)
+  auto general = [&](int o, int oe, int j0, int j1) {
+    for (int c = o, ce; c < oe; c = ce) {
+      const int c0 = std::max(0, c - halo), c1 = std::min(nx, c0 + 64);
+      ce = std::min(oe, c0 + 64 >= nx ? nx : c0 + 64 - halo);
+      const bool cols = plain_cols(c0, c0 + 64), probes = m && count(m->pcol_pref, c0, c1) > 0;
+      for (int j = j0, je; j < j1; j = je) {
+        const int w0 = std::max(0, j - T);
+        je = std::min(j1, w0 + s.RG * s.W >= ny ? ny : w0 + s.RG * s.W - T);
+        fdtd2d::BlockTile t{c0, w0, c, ce, j, je};
+        t.flags = (cols ? 0 : fdtd2d::kBlockX) | fdtd2d::kBlockGeneral;
+        if (!describe(t, s.RG, c1, probes)) return false;
+        out.push_back(t);
+      }
+    }
+    return true;
+  };
+  for (int o = 0, oe; o < nx; o = oe) {
+    const int c0 = o - halo;
+    if (c0 < 0 || !plain_cols(c0, c0 + full_w)) {  // an edge piece, general from top to bottom
+      oe = std::max(0, c0) + 64 >= nx ? nx : std::max(0, c0) + 64 - halo;
+      if (!general(o, oe, 0, ny)) return false;
+      continue;
+    }
+    oe = c0 + full_w - halo;
+    const bool probes = m && count(m->pcol_pref, c0, c0 + full_w) > 0;
+    int g0 = 0;  // rows [g0, j) wait for general tiles
+    const int win = s.R * s.W;
+    for (int j = 0; j < ny;) {
+      const int w0 = j - T;
+      if (w0 >= 1 && plain_rows(w0 - 1, w0 + win) && !events(w0, w0 + win, c0, c0 + full_w)) {
+        if (g0 < j && !general(o, oe, g0, j)) return false;
+        const int je = w0 + win - T;
+        fdtd2d::BlockTile t{c0, w0, o, oe, j, je};
+        if (probes || (m && count(m->lrow_pref, w0, w0 + win))) t.flags = fdtd2d::kBlockCap;
+        describe(t, s.R, c0 + full_w, false);
+        inner.push_back(t);
+        g0 = j = je;
+      } else {
+        // to the next row where an interior tile could start: a general tile further
+        j = std::min(ny, std::max(0, w0) + s.RG * s.W - T);
+      }
+    }
+    if (g0 < ny && !general(o, oe, g0, ny)) return false;
+  }
+  out.insert(out.end(), inner.begin(), inner.end());
+  return true;
+}
+
 // The step kernel hands list positions [x*q + min(x, r), ...) of a G
 // work-group launch (q = G/8, r = G%8) to XCD x in launch order. Work-groups
 // with a Jz update take about 1.6 times as long as those without; moving
@@ -488,6 +588,29 @@ static std::vector<int4> fused_list(const std::vector<int4> &interior, std::vect
     ii += ni;
   }
   return out;
+}
+
+// The block form's shape for a plan, or none where the streaming form is the
+// better one. Measured on MI355X, us per 8-step launch, streaming | {1,4,2,12}
+// | {2,3,3,12} | {1,8,4,8} (C, R, RG, W):
+//   density  256x192  122 | 12.4 | 16.2 | 18.8     1024^2  121 | 22.5 | 22.0 | 23.6
+//            2048^2   123 | 61.5 | 53.9 | 59.3     2896^2  132 |  114 | 98.0 |  108
+//            4096^2   181 |  229 |  193 |  213
+//   table    400^2    206 | 13.3 | 16.9 | 20.6     1024^2  212 | 25.6 | 30.7 | 25.8
+//            2048^2   234 | 68.4 | 89.2 | 64.9     4096^2  323 |  246 |  354 |  224
+// Small grids leave the chip idle, so the least work per wave wins; from
+// about a million cells the fewest recomputed cells (two columns per lane; for
+// the table medium, with ca, cb and Ne in registers, more rows instead). The
+// streaming form moves the state with fewer recomputed cells and overlaps its
+// loads, which wins once it fills the chip (density, from about 3400^2).
+static BlockShape pick_block(const fdtd2d_plan *pl) {
+  if (pl->block == 0 || pl->pooled) return BlockShape();
+  if (pl->block >= 2) return kBlockShapes[pl->block - 2];
+  const long long cells = static_cast<long long>(pl->L.nx) * pl->L.ny;
+  const bool table = pl->a.medium_kind == FDTD2D_MEDIUM_TABLE;
+  if (pl->block < 0 && cells > (table ? 24000000LL : 11500000LL)) return BlockShape();
+  if (cells < 1000000) return kBlockShapes[0];
+  return kBlockShapes[table ? 2 : 1];
 }
 
 // The fused launch is compiled for one and two columns per lane.
@@ -562,6 +685,14 @@ int set_tiling(fdtd2d_plan *pl) {
     lists[1] = std::move(t.lists[1]);
     if (pl->jz_first) order_jz_first(lists[0]);
   }
+  BlockShape bs = pick_block(pl);
+  std::vector<fdtd2d::BlockTile> blocks;
+  if (bs.C && !make_blocks(pl->L.nx, pl->L.ny, pl->a.P, T, bs, &m, blocks)) bs = BlockShape();
+  if (bs.C) {
+    lists[1].clear();
+    lists[0].resize(blocks.size() * (sizeof(fdtd2d::BlockTile) / sizeof(int4)));
+    std::memcpy(lists[0].data(), blocks.data(), blocks.size() * sizeof(fdtd2d::BlockTile));
+  }
   const size_t n = lists[0].size() + lists[1].size();
   int4 *buf = pl->wg_buf;
   if (pl->static_lists) {
@@ -595,7 +726,10 @@ int set_tiling(fdtd2d_plan *pl) {
   commit(a);
   a.tile_list[0] = buf;
   a.tile_list[1] = buf + lists[0].size();
-  a.n_wg[0] = static_cast<int>(lists[0].size()) / fdtd2d::kWavesPerWG;
+  a.block_list = reinterpret_cast<const fdtd2d::BlockTile *>(buf);
+  a.n_blocks = static_cast<int>(blocks.size());
+  pl->bs = bs;
+  a.n_wg[0] = bs.C ? a.n_blocks : static_cast<int>(lists[0].size()) / fdtd2d::kWavesPerWG;
   a.n_wg[1] = static_cast<int>(lists[1].size()) / fdtd2d::kWavesPerWG;
   return FDTD2D_OK;
 }
@@ -1171,7 +1305,7 @@ int fdtd2d_plan_set_option(fdtd2d_plan *pl, const char *name, double value) {
   const int v = static_cast<int>(value);
   // the shape before the change, restored if the new one cannot be set up
   const int oT = pl->T, oband = pl->band, oband_cpml = pl->band_cpml, oC = pl->C, oD = pl->D,
-            ojz = pl->jz_first, ofused = pl->fused;
+            ojz = pl->jz_first, ofused = pl->fused, oblock = pl->block;
   auto retile = [&]() {
     const int rc = set_tiling(pl);
     if (rc) {
@@ -1182,6 +1316,7 @@ int fdtd2d_plan_set_option(fdtd2d_plan *pl, const char *name, double value) {
       pl->D = oD;
       pl->jz_first = ojz;
       pl->fused = ofused;
+      pl->block = oblock;
     }
     return rc;
   };
@@ -1191,25 +1326,35 @@ int fdtd2d_plan_set_option(fdtd2d_plan *pl, const char *name, double value) {
   } else if (n == "band") {
     if (v < 0 || v > pl->L.ny) return set_error(FDTD2D_EINVAL, "band out of range");
     pl->band = v;
+    pl->block = 0;  // options of the streaming form choose it
   } else if (n == "band_cpml") {
     if (v < 0 || v > pl->L.ny) return set_error(FDTD2D_EINVAL, "band_cpml out of range");
     pl->band_cpml = v;
+    pl->block = 0;
   } else if (n == "cols_per_lane") {
     if (v != 1 && v != 2 && v != 4) return set_error(FDTD2D_EINVAL, "cols_per_lane must be 1, 2 or 4");
     pl->C = v;
+    pl->block = 0;
     if (v == 4) pl->D = 1;
     if (v == 2 && pl->D > 2) pl->D = 2;
   } else if (n == "jz_first") {
     if (v != 0 && v != 1) return set_error(FDTD2D_EINVAL, "jz_first must be 0 or 1");
     pl->jz_first = v;
+    pl->block = 0;
   } else if (n == "fused") {
     if (v != 0 && v != 1) return set_error(FDTD2D_EINVAL, "fused must be 0 or 1");
     pl->fused = v;
+    pl->block = 0;
+  } else if (n == "block") {
+    if (v < 0 || v > 1 + static_cast<int>(std::size(kBlockShapes)))
+      return set_error(FDTD2D_EINVAL, "block must be 0 (off), 1 (on) or 2.. (a shape)");
+    pl->block = v;
   } else if (n == "prefetch") {
     const int maxd = pl->C == 1 ? 4 : pl->C == 2 ? 2 : 1;
     if (v != 1 && v != 2 && v != 4) return set_error(FDTD2D_EINVAL, "prefetch must be 1, 2 or 4");
     if (v > maxd) return set_error(FDTD2D_EINVAL, "prefetch depth too large for cols_per_lane");
     pl->D = v;
+    pl->block = 0;
   } else {
     return set_error(FDTD2D_EINVAL, "unknown option " + n);
   }
@@ -1245,6 +1390,7 @@ int fdtd2d_plan_get_info(const fdtd2d_plan *pl, const char *name, double *value)
   else if (n == "prefetch") *value = pl->D;
   else if (n == "jz_first") *value = pl->jz_first;
   else if (n == "fused") *value = fused_launch(pl) ? 1 : 0;
+  else if (n == "block") *value = pl->bs.C ? 1 : 0;
   else if (n == "cus") {
     int ncu = 0;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, pl->device), "hipDeviceGetAttribute");
@@ -1299,7 +1445,8 @@ int fdtd2d_run(fdtd2d_plan *pl, int nsteps) {
     }
     // timing events bracket each kernel alone on its own stream
     if (pl->timing) HIP_TRY(hipEventRecord(e0, pl->stream), "hipEventRecord");
-    hipError_t e = fused_launch(pl) ? fdtd2d::launch_step_fused(pl->a, t, pl->C, pl->D, pl->src, pl->n, pl->stream)
+    hipError_t e = pl->bs.C ? fdtd2d::launch_block(pl->a, pl->bs.C, pl->bs.R, pl->bs.RG, pl->bs.W, t, pl->src, pl->n, pl->stream)
+                   : fused_launch(pl) ? fdtd2d::launch_step_fused(pl->a, t, pl->C, pl->D, pl->src, pl->n, pl->stream)
                              : fdtd2d::launch_step(pl->a, 0, t, pl->C, pl->D, pl->src, pl->n, pl->stream);
     if (e != hipSuccess) return hip_fail(e, "step kernel launch");
     if (pl->timing) {

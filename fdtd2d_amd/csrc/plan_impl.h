@@ -89,6 +89,19 @@ struct TileMasks {
 };
 
 Tiling make_tiling(int nx, int ny, int P, int T, int C, int band, int band_cpml, const TileMasks *m = nullptr);
+// Tiles of the block form (block_device.h), T steps: 64*C columns by R*W rows
+// where the window is clear of strips, ring and events, 64 columns by RG*W
+// rows elsewhere; every cell owned by one tile, general tiles first. False if
+// a wave would hold more than 64 events (that grid keeps the streaming form).
+// Host-only.
+struct BlockShape {
+  int C = 0, R = 0, RG = 0, W = 0;  // C = 0: the streaming form
+};
+// The shapes the block kernels are compiled for (block_kernels.hip).
+constexpr BlockShape kBlockShapes[] = {{1, 4, 2, 12}, {2, 3, 3, 12}, {1, 8, 4, 8}};
+bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMasks *m,
+                 std::vector<fdtd2d::BlockTile> &out);
+
 Layout make_layout(const fdtd2d_problem *p, size_t n_events);
 int hip_fail(hipError_t e, const char *what);
 
@@ -118,6 +131,10 @@ struct fdtd2d_plan {
   int D = 2;     // rows of prefetch per wave (interior kernel); the row loop is unrolled by D
   int band_cpml = 0;               // rows per CPML-class work-group (0: automatic)
   int jz_first = 1;  // interior work-groups with a Jz update first in each XCD's range
+  // block form: -1 by the grid (pick_block), 0 off, 1 on with the shape of the
+  // grid's size, 2 + k shape k of kBlockShapes
+  int block = -1;
+  fdtd2d::detail::BlockShape bs;  // the shape in use (C = 0: the streaming form)
   int fused = 1;     // one kernel per launch over one list (0: interior and CPML-class kernels on two streams)
   double cells_class[2] = {0, 0};  // grid cells owned by interior / CPML-class tiles
   double cells_kind[5] = {0, 0, 0, 0, 0};  // CPML-class cells by kind: general, x strip, y strip, corner, events

@@ -17,7 +17,7 @@ struct Event {
   int32_t i;     // column
   int32_t kind;  // EV_*
   int32_t idx;   // element / detector / component index
-  int32_t pad;
+  int32_t row;
 };
 
 // Everything a step launch reads. Field buffers are ping-ponged: a launch of
@@ -96,10 +96,27 @@ struct StepArgs {
   const int4 *tile_list[2];
   int n_tiles[2];  // entries in use
   int n_wg[2];     // work-groups launched (entries / 4, rounded up)
+  // block form: one entry per work-group
+  const struct BlockTile *block_list;
+  int n_blocks;
   // pool mode: the shot runs in launches g_base, g_base + g_stride, ...; at
   // its d-th such launch (d = (g - g_base) / g_stride) it runs steps
   // n_base + d*tp onwards from buffer set src_base ^ (d & 1)
   int g_base, n_base, src_base, g_stride;
+};
+
+// One tile of the block form (block_device.h), a work-group of W waves. It
+// loads columns from cs on (64 times its columns per lane) of the rows from
+// rs on (wave w those from rs + w*R) and stores [own0, own1) x [r0, r1).
+// kBlockGeneral: the window holds more than interior cells (such a tile has
+// one column per lane and its own R); kBlockX: it reaches an x strip, the ring
+// or a column whose den differ; kBlockCap: an interior tile with RC probes or
+// the processing line. Per wave (bit w): y_waves as kBlockX for its rows,
+// e_waves events or captures, jz_waves plasma or a nonzero Jz, full_waves
+// plasma everywhere.
+constexpr int kBlockX = 1, kBlockGeneral = 2, kBlockCap = 4;
+struct BlockTile {
+  int cs, rs, own0, own1, r0, r1, flags, y_waves, e_waves, jz_waves, full_waves, pad;
 };
 
 // Work queue of the pool kernels, in device memory. items/count: the packed
@@ -168,6 +185,9 @@ hipError_t launch_step(const StepArgs &a, int cls, int T, int C, int D, int src,
 // n_wg[0] work-groups: CPML-class entries flagged kFlagCpml first in each
 // XCD's range, then interior ones). C = 1 or 2.
 hipError_t launch_step_fused(const StepArgs &a, int T, int C, int D, int src, int n0, hipStream_t stream);
+
+// Launches the block kernel (block_list, n_blocks) for T steps.
+hipError_t launch_block(const StepArgs &a, int C, int R, int RG, int W, int T, int src, int n0, hipStream_t stream);
 
 // RC cutoff lines (Dev_RCcalc semantics) for steps n0+1 .. n0+t from the
 // capture of the launch that computed them; one work-group per line.

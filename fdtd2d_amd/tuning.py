@@ -167,8 +167,19 @@ def tune_plan(plan, launches: int = 4, axes=PLAN_AXES, log=None) -> dict:
     band rows, prefetch depth) on the live plan: every trial advances the
     real problem (results do not depend on the shape) and is scored by cell
     updates per second. One untimed trial first (cold caches). Stops when the
-    problem runs out of steps. Leaves the plan at the best shape."""
+    problem runs out of steps. Leaves the plan at the best shape. The axes are
+    the streaming form's; a plan that starts in the block form goes back to it
+    ({"block": 1}) unless one of them beats it."""
     best = {name: int(plan.info(name)) for name, _ in axes}  # the library's default shape first
+    block_rate = 0.0
+    try:
+        block = plan.info("block") > 0
+    except (KeyError, FDTD2DError):
+        block = False
+    if block:
+        _plan_trial(plan, launches)
+        block_rate = _plan_trial(plan, launches)
+        plan.set_option("block", 0)
     _plan_trial(plan, launches)
     best_rate = _plan_trial(plan, launches)
     trials = [(dict(best), best_rate)]
@@ -189,6 +200,9 @@ def tune_plan(plan, launches: int = 4, axes=PLAN_AXES, log=None) -> dict:
             if rate > best_rate:
                 best_rate, best[name] = rate, v
         plan.set_option(name, best[name])
+    if block_rate > best_rate:
+        plan.set_option("block", 1)
+        return {"shape": {"block": 1}, "rate": block_rate, "trials": trials + [({"block": 1}, block_rate)]}
     return {"shape": best, "rate": best_rate, "trials": trials}
 
 

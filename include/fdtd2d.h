@@ -323,13 +323,19 @@ int fdtd2d_plan_set_tblock(fdtd2d_plan *plan, int steps_per_launch);
    CPML-class tile but a few kinds - the general ones, and for the table
    medium the corners - which run in a second kernel beside it only where
    the grid has them; 0: all CPML-class tiles in the second kernel; with 4
-   columns per lane launches are never fused). Results are identical for
-   every choice. */
+   columns per lane launches are never fused), "block" (the form that keeps a
+   tile in registers for a whole launch: 0 off, 1 on, 2 .. 4 on with a given
+   shape; by default on for grids up to about 3400^2 cells (table medium:
+   4900^2) unless a wave would hold more than 64 events; the options above
+   but "tblock" belong to the other form and switch this one off). Results
+   are identical for every choice. */
 int fdtd2d_plan_set_option(fdtd2d_plan *plan, const char *name, double value);
 /* Plan facts by name: "pitch", "tblock", "band", "band_cpml", "ntx", "nty",
    "workgroups", "workgroups_cpml" (work-groups of the second kernel),
    "tile_cols", "bytes", "steps", "cols_per_lane", "prefetch", "jz_first",
-   "fused" (1 when launches are fused), "cells_interior", "cells_cpml",
+   "fused" (1 when launches are fused), "block" (1 when the block form runs;
+   the tile counts and cell shares below describe the other form),
+   "cells_interior", "cells_cpml",
    "tiles_interior", "tiles_cpml", "tiles_nojz" (interior tiles with no Jz
    update), "tiles_plasma_full" (interior tiles whose window has Ne > 0 in
    every cell), "cells_xstrip", "cells_ystrip", "cells_corner",

@@ -1,0 +1,119 @@
+"""The block form of the step kernels (a tile in registers for a whole launch)
+against the FP32 oracle, bit for bit, at the sizes where a tile, a wave's rows
+or the recomputed columns end: windows of 64 and 128 columns, 24, 32, 36 and 64
+rows, grids one cell around them, events in every corner of a tile, RC probes
+and the processing line inside interior tiles, partial launches."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import fdtd2d_amd as F
+from oracle.oracle import Oracle
+
+from helpers import all_state, random_problem
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [2, 3, 4]  # "block" option: the compiled shapes
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+def _check(p, shapes, launches, label, gpu_device):
+    ref = Oracle(p, 32, threads=4)
+    ref.run(p.nsteps)
+    want = all_state(ref, p.npml)
+    extra = {}
+    if p.rc_i.size:
+        extra["rc"] = np.asarray(ref.read_rc())
+    if p.line_size:
+        extra["line"] = np.asarray(ref.read_line())
+    for shape in shapes:
+        with F.Plan(p, gpu_device) as plan:
+            plan.set_option("block", shape)
+            assert plan.info("block") == 1
+            for n in launches:
+                plan.run(n)
+            plan.run(p.nsteps - sum(launches))
+            got = all_state(plan, p.npml)
+            for k in want:
+                assert np.array_equal(_bits(want[k]), _bits(got[k])), f"{label} shape {shape}: {k} differs"
+            if "rc" in extra:
+                assert np.array_equal(plan.read_rc(), extra["rc"]), f"{label} shape {shape}: rc differs"
+            if "line" in extra:
+                assert np.array_equal(_bits(plan.read_line()), _bits(extra["line"])), f"{label} shape {shape}: line"
+
+
+@pytest.mark.parametrize("table", [False, True])
+@pytest.mark.parametrize("nx,ny,npml", [(24, 24, 0), (63, 25, 5), (64, 24, 2), (65, 37, 0), (112, 33, 8), (121, 63, 8),
+                                        (128, 64, 11), (177, 65, 5), (240, 101, 12), (333, 131, 3)])
+def test_edges(gpu_device, nx, ny, npml, table):
+    rng = np.random.default_rng(nx * 1000 + ny + table)
+    p = random_problem(rng, nx=nx, ny=ny, npml=npml, nsteps=21, table=table)
+    _check(p, SHAPES, [8, 1], f"{nx}x{ny} P={npml}", gpu_device)
+
+
+@pytest.mark.parametrize("seed", range(3))
+def test_events_captures_and_odd_den(gpu_device, seed):
+    """Sources that share a cell, detectors on every row of a wave, RC probes
+    and the processing line in interior tiles, den that differs inside."""
+    rng = np.random.default_rng(7100 + seed)
+    p = random_problem(rng, nx=420, ny=300, npml=8, nsteps=27, table=bool(seed & 1), nsrc=6, ndet=40, ncomp=8)
+    p.src_table = p.src_table * 50
+    p.src_i[1], p.src_j[1] = p.src_i[0], p.src_j[0]
+    p.det_i[:20], p.det_j[:20] = 200, 140 + np.arange(20)
+    p.comp_i[0], p.comp_j[0] = p.src_i[0] % 419, p.src_j[0] % 299
+    p.rc_imax = np.array([60, 128, 240, 300], np.int32)
+    p.rc_i = p.rc_imax + np.arange(4, dtype=np.int32)
+    p.rc_jcut, p.rc_level, p.rc_edge0 = 60, 0.07, 1e-3
+    p.line_size, p.line_i0, p.line_j, p.line_begin, p.line_end = 180, 100, 150, 3, 25
+    if seed == 2:
+        p.den_ex, p.den_hy = p.den_ex.copy(), p.den_hy.copy()
+        p.den_ex[230] *= np.float32(1.25)
+        p.den_hy[190:193] *= np.float32(0.8)
+    _check(p, SHAPES, [5, 8], f"seed {seed}", gpu_device)
+
+
+def test_more_events_than_lanes_keeps_the_streaming_form(gpu_device):
+    """A wave with more than 64 events in its rows: the plan stays with the
+    streaming form and still matches."""
+    rng = np.random.default_rng(5)
+    p = random_problem(rng, nx=150, ny=120, npml=6, nsteps=18, table=False, ndet=70)
+    p.det_i[:], p.det_j[:] = 20 + np.arange(70) % 30, 60  # all in the first tile (columns 0..63)
+    ref = Oracle(p, 32)
+    ref.run(p.nsteps)
+    want = all_state(ref, p.npml)
+    with F.Plan(p, gpu_device) as plan:
+        assert plan.info("block") == 0
+        plan.run(p.nsteps)
+        got = all_state(plan, p.npml)
+    for k in want:
+        assert np.array_equal(_bits(want[k]), _bits(got[k])), k
+
+
+def test_default_form_and_options(gpu_device):
+    """Small grids take the block form; an option of the streaming form, or
+    block = 0, leaves it; both forms can follow each other in one run."""
+    rng = np.random.default_rng(6)
+    p = random_problem(rng, nx=200, ny=180, npml=6, nsteps=40, table=False)
+    ref = Oracle(p, 32)
+    ref.run(p.nsteps)
+    want = all_state(ref, p.npml)
+    with F.Plan(p, gpu_device) as plan:
+        assert plan.info("block") == 1
+        plan.run(11)
+        plan.set_option("cols_per_lane", 2)
+        assert plan.info("block") == 0
+        plan.run(13)
+        plan.set_option("block", 1)
+        assert plan.info("block") == 1
+        plan.run(16)
+        got = all_state(plan, p.npml)
+        with pytest.raises(F.FDTD2DError):
+            plan.set_option("block", 9)
+    for k in want:
+        assert np.array_equal(_bits(want[k]), _bits(got[k])), k
