@@ -8,69 +8,57 @@
 namespace fdtd2d {
 namespace {
 
-// RC cutoff lines for the t steps of one launch, in step order (the edge level
-// carries from step to step). Dev_FindMax keeps a value only when a later one
-// is strictly greater, so the maximum is the first of the largest values in
-// scan order (row 0, then rows jcut .. ny-3) and a NaN at row 0 stays; the
-// scan (j from ny-3 down while |Ez| < edge) stops at the largest j >= 1 whose
-// |Ez| is not below the edge, else at 0.
-__global__ void __launch_bounds__(256) rc_kernel(const RcArgs r, int n0, int t) {
-  __shared__ float s_v[256];
-  __shared__ int s_i[256];
-  const int e = blockIdx.x, tid = threadIdx.x;
-  const int pm = r.map[2 * e], ps = r.map[2 * e + 1];
+// RC cutoff lines for the t steps of one launch. Dev_FindMax keeps a value
+// only when a later one is strictly greater, so the maximum is the largest
+// value of row 0 and rows jcut .. ny-3 that is not a NaN, and a NaN at row 0
+// stays; the scan (j from ny-3 down while |Ez| < edge) stops at the largest
+// j >= 1 whose |Ez| is not below the edge, else at 0. Only the edge level
+// carries from step to step: two waves per step find the launch's maxima side
+// by side, one thread runs the edge through them, the waves scan. (Step by
+// step, two block reductions each, a line took 79 us per 8-step launch at
+// 3000 rows, all of it latency, after a step kernel of 45; now 14.6.)
+__global__ void __launch_bounds__(128 * kMaxT) rc_kernel(const RcArgs r, int n0, int t) {
+  __shared__ float s_max[kMaxT][2], s_first[kMaxT], s_edge[kMaxT];
+  __shared__ int s_j[kMaxT][2];
+  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, half = (tid >> 6) & 1, s = tid >> 7;
   const int ny = r.ny;
   const int ncand = 1 + max(0, (ny - 2) - r.jcut);
-  float edge = r.edge[e];
-  for (int s = 1; s <= t; ++s) {
-    const int step = n0 + s;
-    const long long slot = (step - 1) & (kMaxT - 1);
-    const float *cm = r.cap + (slot * r.nprobe + pm) * ny;
-    const float *cs = r.cap + (slot * r.nprobe + ps) * ny;
-    // (value, candidate index): larger value wins, equal values the earlier
-    float bv = 0.f;
-    int bi = 0x7fffffff;
-    for (int q = tid; q < ncand; q += blockDim.x) {
-      const float v = q == 0 ? cm[0] : cm[r.jcut + q - 1];
-      if (v != v) continue;  // NaN never replaces (row 0 handled below)
-      if (bi == 0x7fffffff || v > bv || (v == bv && q < bi)) {
-        bv = v;
-        bi = q;
-      }
+  const long long slot = (n0 + s) & (kMaxT - 1);
+  if (s < t) {
+    const float *cm = r.cap + (slot * r.nprobe + r.map[2 * e]) * ny;
+    float m = -INFINITY;
+#pragma unroll 8
+    for (int q = half * 64 + lane; q < ncand; q += 128) m = fmaxf(m, q == 0 ? cm[0] : cm[r.jcut + q - 1]);
+    for (int w = 32; w > 0; w >>= 1) m = fmaxf(m, __shfl_xor(m, w));
+    if (lane == 0) {
+      s_max[s][half] = m;
+      if (half == 0) s_first[s] = cm[0];
     }
-    s_v[tid] = bv;
-    s_i[tid] = bi;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-      if (tid < w) {
-        const float ov = s_v[tid + w];
-        const int oi = s_i[tid + w];
-        if (oi != 0x7fffffff &&
-            (s_i[tid] == 0x7fffffff || ov > s_v[tid] || (ov == s_v[tid] && oi < s_i[tid]))) {
-          s_v[tid] = ov;
-          s_i[tid] = oi;
-        }
-      }
-      __syncthreads();
-    }
-    const float c0 = cm[0];
-    const float temp = c0 != c0 ? c0 : s_v[0];
-    __syncthreads();
-    const float et = temp * r.level;
-    if (et > edge) edge = et;
-    int bj = 0;
-    for (int j = 1 + tid; j <= ny - 3; j += blockDim.x)
-      if (!(fabsf(cs[j]) < edge)) bj = max(bj, j);
-    s_i[tid] = bj;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-      if (tid < w) s_i[tid] = max(s_i[tid], s_i[tid + w]);
-      __syncthreads();
-    }
-    if (tid == 0) r.spd[static_cast<long long>(step) * r.nrc + e] = s_i[0];
-    __syncthreads();
   }
-  if (tid == 0) r.edge[e] = edge;
+  __syncthreads();
+  if (tid == 0) {
+    float edge = r.edge[e];
+    for (int k = 0; k < t; ++k) {
+      const float c0 = s_first[k];
+      const float et = (c0 != c0 ? c0 : fmaxf(s_max[k][0], s_max[k][1])) * r.level;
+      if (et > edge) edge = et;
+      s_edge[k] = edge;
+    }
+    r.edge[e] = edge;
+  }
+  __syncthreads();
+  if (s < t) {
+    const float *cs = r.cap + (slot * r.nprobe + r.map[2 * e + 1]) * ny;
+    const float edge = s_edge[s];
+    int bj = 0;
+#pragma unroll 8
+    for (int j = 1 + half * 64 + lane; j <= ny - 3; j += 128)
+      if (!(fabsf(cs[j]) < edge)) bj = j;  // j grows: the last one is the largest
+    for (int w = 32; w > 0; w >>= 1) bj = max(bj, __shfl_xor(bj, w));
+    if (lane == 0) s_j[s][half] = bj;
+  }
+  __syncthreads();
+  if (tid < t) r.spd[static_cast<long long>(n0 + 1 + tid) * r.nrc + e] = max(s_j[tid][0], s_j[tid][1]);
 }
 
 template <int T, int C, int D, int MODE>
@@ -105,7 +93,7 @@ hipError_t launch_cd(const StepArgs &a, int T, int src, int n0, hipStream_t s) {
 hipError_t launch_rc(const RcArgs &r, int n0, int t, hipStream_t stream) {
   if (r.nrc <= 0 || t <= 0) return hipSuccess;
   if (t > kMaxT) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(rc_kernel, dim3(r.nrc), dim3(256), 0, stream, r, n0, t);
+  hipLaunchKernelGGL(rc_kernel, dim3(r.nrc), dim3(128 * kMaxT), 0, stream, r, n0, t);
   return hipGetLastError();
 }
 

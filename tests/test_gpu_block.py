@@ -117,3 +117,27 @@ def test_default_form_and_options(gpu_device):
             plan.set_option("block", 9)
     for k in want:
         assert np.array_equal(_bits(want[k]), _bits(got[k])), k
+
+
+@pytest.mark.parametrize("ny", [66, 133, 300])
+@pytest.mark.parametrize("jcut", [0, 9, 64, 500])
+def test_rc_candidates(gpu_device, ny, jcut):
+    """The RC maximum over row 0 and rows jcut .. ny-3 (none past the grid),
+    the edge carried over launches of 8, 3 and the rest, with a NaN at row 0 of
+    one probe column."""
+    rng = np.random.default_rng(ny + jcut)
+    p = random_problem(rng, nx=140, ny=ny, npml=5, nsteps=30, table=True)
+    p.src_table = p.src_table * 50
+    p.rc_imax = np.array([50, 80, 101], np.int32)
+    p.rc_i = p.rc_imax + np.int32(2)
+    p.rc_jcut, p.rc_level, p.rc_edge0 = jcut, 0.07, 1e-4
+    ez = np.zeros((ny, 140), np.float32)
+    ez[0, 80] = np.nan  # a ring cell: never updated
+    ref = Oracle(p, 32)
+    ref.write_field(F.EZ, ez)
+    ref.run(p.nsteps)
+    with F.Plan(p, gpu_device) as plan:
+        plan.write_field(F.EZ, ez)
+        for n in (8, 3, 19):
+            plan.run(n)
+        assert np.array_equal(plan.read_rc(), np.asarray(ref.read_rc()))
