@@ -71,6 +71,10 @@ def _descend(pool: Pool, start: dict, axes, launches_per_trial: int, trials: lis
     return best, best_rate
 
 
+def _block_form(pool) -> bool:
+    return isinstance(pool, Pool) and pool.info("block") > 0
+
+
 def autotune(pool: Pool, launches_per_trial: int = 4, axes=TUNE_AXES, log=None, margin: float = 0.95) -> dict:
     """Picks the launch shape for the shots now in the pool; returns it with
     the score of every trial. A coordinate descent with one kernel per tile
@@ -80,6 +84,13 @@ def autotune(pool: Pool, launches_per_trial: int = 4, axes=TUNE_AXES, log=None, 
     Stops early when the pool runs out of work."""
     trials = []
     found = []
+    if pool.info("running") > 0 and _block_form(pool):
+        # the axes below are the streaming form's; the pool goes back to the
+        # block form it started in unless one of them beats it
+        block = {"tblock": int(pool.info("tblock")), "block": 1}
+        _trial(pool, launches_per_trial)
+        found.append((block, _trial(pool, launches_per_trial)))
+        trials.append(found[0])
     if pool.info("running") > 0:
         start = {"fused": 0, **{name: values[0] for name, values in axes}}
         for name, value in start.items():
@@ -89,14 +100,14 @@ def autotune(pool: Pool, launches_per_trial: int = 4, axes=TUNE_AXES, log=None, 
         _trial(pool, launches_per_trial)
         found.append(_descend(pool, start, axes, launches_per_trial, trials, log))
     if found and pool.info("running") > 0:
-        shape = {**found[0][0], "fused": 1}
+        shape = {**found[-1][0], "fused": 1}
         for name, value in shape.items():
             pool.set_option(name, value)
         rate = _trial(pool, launches_per_trial)
         trials.append((dict(shape), rate))
         if log:
-            log(f"autotune fused=1 at that shape: {rate / 1e9:.1f} Gcell/s (best {found[0][1] / 1e9:.1f})")
-        if rate >= margin * found[0][1]:
+            log(f"autotune fused=1 at that shape: {rate / 1e9:.1f} Gcell/s (best {found[-1][1] / 1e9:.1f})")
+        if rate >= margin * found[-1][1]:
             found.append(_descend(pool, shape, axes, launches_per_trial, trials, log))
     if not found:
         return {"shape": {}, "rate": 0.0, "trials": trials}

@@ -41,6 +41,15 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
+// The step loop's barrier. The wait for the wave's own LDS writes is spelled
+// out: the compiler (ROCm 7.2) dropped the one that the barrier's release
+// fence stands for from loops whose header holds the barrier, and a wave then
+// read a neighbour's row before it had arrived (one launch in thousands).
+__device__ __forceinline__ void step_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 // One wave's part of a tile. JZ as in the streaming form (0: no plasma and no
 // Jz in the wave's rows, 2: all of it plasma); with K != 0, where JZ is 1,
 // `jz_on` says whether there is any (uniform). Every readlane below is reached
@@ -175,7 +184,7 @@ __device__ __forceinline__ void block_wave(const StepArgs &a, const float4 *lut_
     const int e0 = cld(a.ev_off, max(0, min(rb, ny))), e1 = cld(a.ev_off, max(0, min(rb + R, ny)));
     if (e0 < e1) {
       // gathered through the 128 words of LDS that the wave publishes to
-      int *box = reinterpret_cast<int *>(sh + wave * 2 * 64);
+      float *box = sh + wave * 2 * 64;
       int n = 0;
       for (int eb = e0; eb < e1; eb += 64) {
         rec_v4i v = {-1, 0, 0, 0};
@@ -184,16 +193,16 @@ __device__ __forceinline__ void block_wave(const StepArgs &a, const float4 *lut_
         const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
         const int at = n + __builtin_amdgcn_mbcnt_hi(m >> 32, __builtin_amdgcn_mbcnt_lo(m, 0));
         if (in && at < 64) {
-          box[2 * at] = (v.x - t.cs) | v.y << 8 | (v.w - rb) << 16;
-          box[2 * at + 1] = v.z;
+          box[2 * at] = __int_as_float((v.x - t.cs) | v.y << 8 | (v.w - rb) << 16);
+          box[2 * at + 1] = __int_as_float(v.z);
         }
         n += __builtin_popcountll(m);
       }
       if (lane < n) {
-        const int w = box[2 * lane], kind = (w >> 8) & 255;
+        const int w = __float_as_int(box[2 * lane]), kind = (w >> 8) & 255;
         ev_lane = w & 255;
         ev_row = w >> 16;
-        ev_idx = box[2 * lane + 1];
+        ev_idx = __float_as_int(box[2 * lane + 1]);
         ev_is_src = kind == EV_SRC;
         const bool mine = rb + ev_row >= t.r0 && rb + ev_row < t.r1 && t.cs + ev_lane >= t.own0 && t.cs + ev_lane < t.own1;
         ev_det = mine && kind == EV_DET;
@@ -304,7 +313,7 @@ __device__ __forceinline__ void block_wave(const StepArgs &a, const float4 *lut_
   };
 
   for (int s = 0; s < T; ++s) {
-    __syncthreads();
+    step_barrier();
     // rows whose state after this step the stored rows depend on; a wave with
     // none of them is done (it still takes part in the barriers)
     const int left = T - 1 - s;
@@ -482,7 +491,7 @@ __device__ __forceinline__ void block_inner(const StepArgs &a, const float4 *lut
     }
   };
   for (int s = 0; s < T; ++s) {
-    __syncthreads();
+    step_barrier();
     const int left = T - 1 - s;
     if (rb + R <= t.r0 - left || rb >= t.r1 + left) continue;
     const int buf = (s & 1) * kBuf;
@@ -560,20 +569,33 @@ __device__ __forceinline__ void run_block(const StepArgs &a, const float4 *lut_s
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool x = t.flags & kBlockX, y = t.y_waves >> wave & 1, e = t.e_waves >> wave & 1;
   const bool jz = t.jz_waves >> wave & 1, full = t.full_waves >> wave & 1;
-#define FDTD2D_WAVE(K) block_wave<RG, W, K, MED, 1>(a, lut_s, sh, src, n0, T, t, wave, jz)
-#define FDTD2D_INNER(JZ, CAP) block_inner<C, R, W, MED, JZ, CAP>(a, lut_s, sh, src, n0, T, t, wave)
+  // The marks keep the compiler from merging the forms' common beginnings and
+  // ends (their loads and stores would then hold every form's state at once:
+  // 95 instead of 67 registers at C = 2, R = 4).
+#define FDTD2D_WAVE(K)                                                    \
+  {                                                                       \
+    asm volatile("; general %0" ::"n"(K));                                \
+    block_wave<RG, W, K, MED, 1>(a, lut_s, sh, src, n0, T, t, wave, jz);  \
+    asm volatile("; end general %0" ::"n"(K));                            \
+  }
+#define FDTD2D_INNER(JZ, CAP)                                             \
+  {                                                                       \
+    asm volatile("; interior %0" ::"n"(2 * JZ + CAP));                    \
+    block_inner<C, R, W, MED, JZ, CAP>(a, lut_s, sh, src, n0, T, t, wave); \
+    asm volatile("; end interior %0" ::"n"(2 * JZ + CAP));                \
+  }
   if (t.flags & kBlockGeneral) {
-    if (e) FDTD2D_WAVE(kGeneral);
-    else if (x && y) FDTD2D_WAVE(kX | kY);
-    else if (x) FDTD2D_WAVE(kX);
-    else if (y) FDTD2D_WAVE(kY);
-    else FDTD2D_WAVE(0);
+    if (e) FDTD2D_WAVE(kGeneral)
+    else if (x && y) FDTD2D_WAVE(kX | kY)
+    else if (x) FDTD2D_WAVE(kX)
+    else if (y) FDTD2D_WAVE(kY)
+    else FDTD2D_WAVE(0)
     return;
   }
-  if (t.flags & kBlockCap) FDTD2D_INNER(1, true);
-  else if (!jz) FDTD2D_INNER(0, false);
-  else if (MED == kDensity && full) FDTD2D_INNER(2, false);
-  else FDTD2D_INNER(1, false);
+  if (t.flags & kBlockCap) FDTD2D_INNER(1, true)
+  else if (!jz) FDTD2D_INNER(0, false)
+  else if (MED == kDensity && full) FDTD2D_INNER(2, false)
+  else FDTD2D_INNER(1, false)
 #undef FDTD2D_WAVE
 #undef FDTD2D_INNER
 }
@@ -593,6 +615,7 @@ __device__ __forceinline__ BlockTile load_block(const BlockTile *list, int pos) 
   t.e_waves = c.x;
   t.jz_waves = c.y;
   t.full_waves = c.z;
+  t.slot = c.w;
   return t;
 }
 
@@ -610,6 +633,27 @@ __global__ void __launch_bounds__(64 * W, O) block_kernel(const StepArgs args, i
   const int G = gridDim.x, b = blockIdx.x;
   const int xcd = b & 7, q = G >> 3, rr = G & 7;
   run_block<C, R, RG, W, MED>(a, lut_s, sh, src, n0, T, load_block(a.block_list, xcd * q + min(xcd, rr) + (b >> 3)));
+}
+
+// The tiles of a pool's shots (list 0 of q), launch k of a chunk.
+template <int C, int R, int RG, int W, int MED, int O>
+__global__ void __launch_bounds__(64 * W, O)
+    block_pool_kernel(const StepArgs *__restrict__ descs, const PoolQueue *__restrict__ q, int k, int tp, int T) {
+  __shared__ float4 lut_s[MED == kTable ? 256 : 1];
+  __shared__ float sh[2 * W * 2 * 64 * C];
+  const int G = q->count[0], b = blockIdx.x;
+  if (b >= G) return;
+  const int xcd = b & 7, n = G >> 3, rr = G & 7;
+  const BlockTile t =
+      load_block(reinterpret_cast<const BlockTile *>(q->items[0]), xcd * n + min(xcd, rr) + (b >> 3));
+  const StepArgs &a = *(const StepArgs *)((cargs_ptr)(descs + t.slot));
+  if constexpr (MED == kTable) {
+    for (int m = threadIdx.x; m < a.nmat; m += blockDim.x) lut_s[m] = gload4(a.lut, m);
+    __syncthreads();
+  }
+  const int g = __builtin_amdgcn_readfirstlane(q->g) + k;
+  const int dg = a.g_stride == 1 ? g - a.g_base : (g - a.g_base) / a.g_stride;
+  run_block<C, R, RG, W, MED>(a, lut_s, sh, a.src_base ^ (dg & 1), a.n_base + dg * tp, T, t);
 }
 
 }  // namespace

@@ -590,36 +590,40 @@ static std::vector<int4> fused_list(const std::vector<int4> &interior, std::vect
   return out;
 }
 
+// Measured on MI355X, us per 8-step launch, streaming | {1,4,2,12} |
+// {1,6,3,12} | {2,4,3,12} | {1,8,4,8} (C, R, RG, W):
+//   density  256x192  122 | 12.4 | 16.3 | 16.3 | 18.9    611x1237 121 | 19.3 | 19.8 | 22.5 | 22.2
+//            1024^2   121 | 22.5 | 20.0 | 23.3 | 23.4    1448^2   125 | 35.2 | 33.2 | 32.0 | 35.4
+//            2048^2   123 | 59.4 | 57.7 | 54.1 | 58.4    4096^2   182 |  223 |  207 |  188 |  212
+//   table    400^2    206 | 13.3 |    - |    - | 20.6    1024^2   212 | 25.6 |    - |    - | 25.8
+//            2048^2   234 | 68.4 |    - |    - | 64.9    4096^2   323 |  246 |    - |    - |  224
+// Small grids leave the chip idle, so the least work per wave wins; larger
+// ones fill it, and the fewest recomputed cells win (more rows per wave, then
+// two columns per lane).
+BlockShape block_shape_for(double cells, int medium_kind) {
+  if (medium_kind == FDTD2D_MEDIUM_TABLE) return kBlockShapes[cells < 1.1e6 ? 2 : 3];
+  return kBlockShapes[cells < 7.5e5 ? 2 : cells < 1.5e6 ? 1 : 0];
+}
+
 // The block form's shape for a plan, or none where the streaming form is the
-// better one. Measured on MI355X, us per 8-step launch, streaming | {1,4,2,12}
-// | {2,3,3,12} | {1,8,4,8} (C, R, RG, W):
-//   density  256x192  122 | 12.4 | 16.2 | 18.8     1024^2  121 | 22.5 | 22.0 | 23.6
-//            2048^2   123 | 61.5 | 53.9 | 59.3     2896^2  132 |  114 | 98.0 |  108
-//            4096^2   181 |  229 |  193 |  213
-//   table    400^2    206 | 13.3 | 16.9 | 20.6     1024^2  212 | 25.6 | 30.7 | 25.8
-//            2048^2   234 | 68.4 | 89.2 | 64.9     4096^2  323 |  246 |  354 |  224
-// Small grids leave the chip idle, so the least work per wave wins; from
-// about a million cells the fewest recomputed cells (two columns per lane; for
-// the table medium, with ca, cb and Ne in registers, more rows instead). The
-// streaming form moves the state with fewer recomputed cells and overlaps its
-// loads, which wins once it fills the chip (density, from about 3400^2).
+// better one: that moves the state with fewer recomputed cells (four columns
+// in five stored and eleven rows in twelve, against seven in eight and two in
+// three) but its launch lasts as long as its slowest wave, 120 us, so it wins
+// once it fills the chip (density: 2896^2 132 against 95 us, 4096^2 182
+// against 188, 8192^2 638 against 706; table 4096^2 323 against 224).
 static BlockShape pick_block(const fdtd2d_plan *pl) {
   if (pl->block == 0 || pl->pooled) return BlockShape();
   if (pl->block >= 2) return kBlockShapes[pl->block - 2];
-  const long long cells = static_cast<long long>(pl->L.nx) * pl->L.ny;
+  const double cells = static_cast<double>(pl->L.nx) * pl->L.ny;
   const bool table = pl->a.medium_kind == FDTD2D_MEDIUM_TABLE;
-  if (pl->block < 0 && cells > (table ? 24000000LL : 11500000LL)) return BlockShape();
-  if (cells < 1000000) return kBlockShapes[0];
-  return kBlockShapes[table ? 2 : 1];
+  if (pl->block < 0 && cells > (table ? 2.4e7 : 1.5e7)) return BlockShape();
+  return block_shape_for(cells, pl->a.medium_kind);
 }
 
 // The fused launch is compiled for one and two columns per lane.
 static bool fused_launch(const fdtd2d_plan *pl) { return pl->fused && pl->C <= 2; }
 
-// Builds the tile lists of the plan's launch shape and puts them where the
-// step kernels read them. Nothing of the plan changes unless this succeeds.
-int set_tiling(fdtd2d_plan *pl) {
-  const int T = pl->T > 0 ? pl->T : kDefaultT;
+static TileMasks masks_of(const fdtd2d_plan *pl) {
   TileMasks m;
   m.srow_pref = pl->srow_pref.data();
   m.scol_pref = pl->scol_pref.data();
@@ -635,6 +639,23 @@ int set_tiling(fdtd2d_plan *pl) {
   m.jz_hi = pl->jz_hi.data();
   m.ev = pl->ev_cells.data();
   m.nev = pl->ev_cells.size();
+  return m;
+}
+
+bool block_tiles(fdtd2d_plan *pl, const BlockShape &s, int T) {
+  if (pl->blocks_T == T && pl->blocks_shape == s) return !pl->blocks.empty();
+  const TileMasks m = masks_of(pl);
+  if (!make_blocks(pl->L.nx, pl->L.ny, pl->a.P, T, s, &m, pl->blocks)) pl->blocks.clear();
+  pl->blocks_shape = s;
+  pl->blocks_T = T;
+  return !pl->blocks.empty();
+}
+
+// Builds the tile lists of the plan's launch shape and puts them where the
+// step kernels read them. Nothing of the plan changes unless this succeeds.
+int set_tiling(fdtd2d_plan *pl) {
+  const int T = pl->T > 0 ? pl->T : kDefaultT;
+  const TileMasks m = masks_of(pl);
   Tiling t = make_tiling(pl->L.nx, pl->L.ny, pl->a.P, T, pl->C, pl->band, pl->band_cpml, &m);
   // the geometry and counts the kernels and the info calls read
   auto commit = [&](fdtd2d::StepArgs &a) {
@@ -1419,8 +1440,9 @@ int fdtd2d_plan_set_option(fdtd2d_plan *pl, const char *name, double value) {
     pl->fused = v;
     pl->block = 0;
   } else if (n == "block") {
-    if (v < 0 || v > 1 + static_cast<int>(std::size(kBlockShapes)))
-      return set_error(FDTD2D_EINVAL, "block must be 0 (off), 1 (on) or 2.. (a shape)");
+    if (v < 0 || v > 1 + static_cast<int>(std::size(kBlockShapes)) ||
+        (v >= 2 && v - 2 < kBlockDensityOnly && pl->a.medium_kind == FDTD2D_MEDIUM_TABLE))
+      return set_error(FDTD2D_EINVAL, "block must be 0 (off), 1 (on) or 2 .. 5 (a shape; table medium: 4 or 5)");
     pl->block = v;
   } else if (n == "prefetch") {
     const int maxd = pl->C == 1 ? 4 : pl->C == 2 ? 2 : 1;

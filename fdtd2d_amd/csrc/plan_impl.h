@@ -96,9 +96,15 @@ Tiling make_tiling(int nx, int ny, int P, int T, int C, int band, int band_cpml,
 // Host-only.
 struct BlockShape {
   int C = 0, R = 0, RG = 0, W = 0;  // C = 0: the streaming form
+  bool operator==(const BlockShape &o) const { return C == o.C && R == o.R && RG == o.RG && W == o.W; }
 };
-// The shapes the block kernels are compiled for (block_kernels.hip).
-constexpr BlockShape kBlockShapes[] = {{1, 4, 2, 12}, {2, 3, 3, 12}, {1, 8, 4, 8}};
+// The shapes the block kernels are compiled for (block_kernels.hip): the
+// first two for the density medium only (with ca and cb in registers too they
+// would spill).
+constexpr BlockShape kBlockShapes[] = {{2, 4, 3, 12}, {1, 6, 3, 12}, {1, 4, 2, 12}, {1, 8, 4, 8}};
+constexpr int kBlockDensityOnly = 2;
+// The shape for grids of `cells` cells in all advanced by one launch.
+BlockShape block_shape_for(double cells, int medium_kind);
 bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMasks *m,
                  std::vector<fdtd2d::BlockTile> &out);
 
@@ -135,6 +141,10 @@ struct fdtd2d_plan {
   // grid's size, 2 + k shape k of kBlockShapes
   int block = -1;
   fdtd2d::detail::BlockShape bs;  // the shape in use (C = 0: the streaming form)
+  // pooled: the shot's block tiles at a shape and step count (block_tiles)
+  std::vector<fdtd2d::BlockTile> blocks;
+  fdtd2d::detail::BlockShape blocks_shape;
+  int blocks_T = 0;
   int fused = 1;     // one kernel per launch over one list (0: interior and CPML-class kernels on two streams)
   double cells_class[2] = {0, 0};  // grid cells owned by interior / CPML-class tiles
   double cells_kind[5] = {0, 0, 0, 0, 0};  // CPML-class cells by kind: general, x strip, y strip, corner, events
@@ -191,6 +201,9 @@ int create_plan(const fdtd2d_problem *p, int device, bool pooled, hipStream_t st
 // Bytes create_plan needs for p (the plan's own allocation).
 size_t plan_bytes(const fdtd2d_problem *p);
 int set_tiling(fdtd2d_plan *pl);
+// A pooled shot's block tiles for T steps, made once per shape; false if it
+// cannot take that shape.
+bool block_tiles(fdtd2d_plan *pl, const BlockShape &s, int T);
 int current_T(const fdtd2d_plan *pl);
 
 }  // namespace detail

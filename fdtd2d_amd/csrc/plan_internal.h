@@ -113,10 +113,10 @@ struct StepArgs {
 // or a column whose den differ; kBlockCap: an interior tile with RC probes or
 // the processing line. Per wave (bit w): y_waves as kBlockX for its rows,
 // e_waves events or captures, jz_waves plasma or a nonzero Jz, full_waves
-// plasma everywhere.
+// plasma everywhere. slot: a pool's shot.
 constexpr int kBlockX = 1, kBlockGeneral = 2, kBlockCap = 4;
 struct BlockTile {
-  int cs, rs, own0, own1, r0, r1, flags, y_waves, e_waves, jz_waves, full_waves, pad;
+  int cs, rs, own0, own1, r0, r1, flags, y_waves, e_waves, jz_waves, full_waves, slot;
 };
 
 // Work queue of the pool kernels, in device memory. items/count: the packed
@@ -214,6 +214,11 @@ hipError_t launch_pool(const StepArgs *descs, PoolQueue *q, int k, int tp, int c
 // The C = 2 forms of classes 0 and 2 (their own translation unit).
 hipError_t launch_pool_c2(const StepArgs *descs, PoolQueue *q, int k, int tp, int cls, int T, int D,
                           int medium_kind, int grid, hipStream_t stream);
+// The block form of a pool launch: list 0 holds BlockTile entries (count 0 of
+// them); grid >= that count (work-groups past it end at once, so that a
+// captured launch serves lists of other lengths).
+hipError_t launch_pool_block(const StepArgs *descs, PoolQueue *q, int k, int tp, int C, int R, int RG, int W, int T,
+                             int medium_kind, int grid, hipStream_t stream);
 // Resets the tickets of launches [0, nk) and adds dg to q->g (one wave).
 hipError_t launch_pool_tick(PoolQueue *q, int nk, int dg, hipStream_t stream);
 // Points q at new lists (g >= 0 also sets q->g), in stream order.

@@ -41,6 +41,16 @@ namespace {
 
 constexpr size_t kArenaAlign = 256;
 
+// Cells up to which a launch runs in the block form (block_shape). Measured on
+// MI355X, us per 8-step launch, streaming | block:
+//   density  896^2 shots       4: 329 |  56   16: 343 | 177   32: 442 | 335   64 (51 Mcells): 684 | 650
+//            256..2048 uneven  4: 353 |  78   16: 382 | 272   32: 619 | 578   48 (70 Mcells): 856 | 839
+//            300..600 uneven   4: 313 |  26   16: 339 |  74   64: 367 | 244   (64 of 256..2048, 92 Mcells: 1036 | 1160)
+//   table    896^2 shots       4: 340 |  56   64: 748 | 729   48 of 256..2048: 939 | 934
+// However few its tiles, a streaming launch lasts as long as its slowest wave;
+// with many it keeps every wave busy and recomputes fewer cells.
+constexpr double kPoolBlockCells = 7e7;
+
 // First-fit allocator over one device allocation.
 struct Arena {
   char *base = nullptr;
@@ -132,6 +142,8 @@ struct fdtd2d_pool {
   // (defaults: the shape the autotuner picks for mixed shot sizes)
   int T = 8, band = 128, band_cpml = 64, D = 1, C = 1;
   int wg_per_cu = 3, wg_per_cu_cpml = 2;
+  // block form: -1 by the cells of the shots a launch advances (block_shape), 0 off, 1 on
+  int block = -1;
   int fused = 0;  // 0: one kernel per tile class on two streams; 1: one kernel, CPML-class work first
   int chunk = 8;  // launches per captured graph; 0 = no graphs
   int medium_kind = -1;
@@ -159,11 +171,13 @@ struct fdtd2d_pool {
     int last_g = -1;  // last pool launch that read it
     bool valid = false;
     std::vector<int> set;  // slots whose tiles it holds
+    BlockShape bs;         // in the block form of this shape (C = 0: the streaming form)
     int count[fdtd2d::kPoolLists] = {0, 0, 0};
   } bufs[kListBufs];
   int nbufs = kListBufs;
   int cur = 0;
   int main_count[fdtd2d::kPoolLists] = {0, 0, 0};  // work-groups per list of the current main lists
+  BlockShape main_bs;                              // and their form
   // tail lists: one copy per tail group, taken in turn; a launch has at most
   // T - 1 <= 7 groups, so a copy is reused only after launches whose
   // completion events exist, and is waited for through them
@@ -233,8 +247,17 @@ void append_shot(const fdtd2d_pool *pp, int s, std::vector<int4> *lists) {
   }
 }
 
+// The block form's shape for launches of `slots`, or none (kPoolBlockCells;
+// never by itself while slicing, which gives the streaming form bands of its own).
+BlockShape block_shape(const fdtd2d_pool *pp, const std::vector<int> &slots, int T);
+
+// Launch size of n block tiles: rounded up, so that a captured graph serves
+// sets of about the same size.
+int block_grid(int n) { return (n + 127) / 128 * 128; }
+
 // Copies the lists to device buffers d[], growing them as needed.
-int upload_lists(const std::vector<int4> *lists, int4 **d, size_t *cap, int count[fdtd2d::kPoolLists]) {
+int upload_lists(const std::vector<int4> *lists, const BlockShape &bs, int4 **d, size_t *cap,
+                 int count[fdtd2d::kPoolLists]) {
   bool moved = false;
   for (int c = 0; c < fdtd2d::kPoolLists; ++c) {
     int rc = grow(d[c], cap[c], std::max<size_t>(lists[c].size(), 4), moved);
@@ -242,9 +265,30 @@ int upload_lists(const std::vector<int4> *lists, int4 **d, size_t *cap, int coun
     if (!lists[c].empty())
       HIP_TRY(hipMemcpy(d[c], lists[c].data(), lists[c].size() * sizeof(int4), hipMemcpyHostToDevice),
               "hipMemcpy pool lists");
-    count[c] = static_cast<int>(lists[c].size() / fdtd2d::kWavesPerWG);
+    count[c] = static_cast<int>(lists[c].size() / (bs.C ? sizeof(fdtd2d::BlockTile) / sizeof(int4)
+                                                          : static_cast<size_t>(fdtd2d::kWavesPerWG)));
   }
   return FDTD2D_OK;
+}
+
+// The lists of `slots` in the form `bs`.
+void build_lists(const fdtd2d_pool *pp, const std::vector<int> &slots, const BlockShape &bs,
+                 std::vector<int4> *lists) {
+  if (!bs.C) {
+    for (int s : slots) append_shot(pp, s, lists);
+    return;
+  }
+  // every shot's general tiles, the slower ones, before the interior ones
+  std::vector<fdtd2d::BlockTile> all;
+  for (int pass = 0; pass < 2; ++pass)
+    for (int s : slots)
+      for (fdtd2d::BlockTile t : pp->shots[s].pl->blocks) {
+        if (((t.flags & fdtd2d::kBlockGeneral) != 0) != (pass == 0)) continue;
+        t.slot = s;
+        all.push_back(t);
+      }
+  lists[0].resize(all.size() * (sizeof(fdtd2d::BlockTile) / sizeof(int4)));
+  std::memcpy(lists[0].data(), all.data(), all.size() * sizeof(fdtd2d::BlockTile));
 }
 
 // Makes ring buffer `nb` (holding the lists of `slots`) the current lists.
@@ -255,6 +299,10 @@ int use_lists(fdtd2d_pool *pp, int nb, const std::vector<int> &slots) {
   // a captured graph holds the leftover kernel's grid (none when list 2 is empty)
   const int gc = pp->ncu * pp->wg_per_cu_cpml;
   if (std::min(gc, b.count[2]) != std::min(gc, pp->main_count[2])) pp->graph_valid = false;
+  // and the form, with the block form's grid
+  if (!(b.bs == pp->main_bs) || (b.bs.C && block_grid(b.count[0]) != block_grid(pp->main_count[0])))
+    pp->graph_valid = false;
+  pp->main_bs = b.bs;
   for (int c = 0; c < fdtd2d::kPoolLists; ++c) pp->main_count[c] = b.count[c];
   pp->cur = nb;
   pp->main_set = slots;
@@ -270,7 +318,8 @@ int rebuild_main(fdtd2d_pool *pp, const std::vector<int> &slots) {
     }
   const auto t0 = std::chrono::steady_clock::now();
   std::vector<int4> lists[fdtd2d::kPoolLists];
-  for (int s : slots) append_shot(pp, s, lists);
+  const BlockShape bs = block_shape(pp, slots, pp->T);
+  build_lists(pp, slots, bs, lists);
   bool valid[fdtd2d_pool::kListBufs];
   int last_g[fdtd2d_pool::kListBufs];
   for (int i = 0; i < pp->nbufs; ++i) {
@@ -283,9 +332,10 @@ int rebuild_main(fdtd2d_pool *pp, const std::vector<int> &slots) {
   retire(pp, b.last_g + 1);  // launches that read this buffer have finished
   pp->blocked_s += seconds_since(tw);
   b.valid = false;
-  int rc = upload_lists(lists, b.d, b.cap, b.count);
+  int rc = upload_lists(lists, bs, b.d, b.cap, b.count);
   if (rc) return rc;
   b.set = slots;
+  b.bs = bs;
   b.valid = true;
   if ((rc = use_lists(pp, nb, slots))) return rc;
   pp->rebuilds++;
@@ -300,6 +350,25 @@ void invalidate_lists(fdtd2d_pool *pp) {
 }
 
 bool slicing(const fdtd2d_pool *pp) { return pp->slice_every > 1 && pp->slice_cells > 0; }
+
+BlockShape block_shape(const fdtd2d_pool *pp, const std::vector<int> &slots, int T) {
+  if (pp->block == 0 || slots.empty() || (pp->block < 0 && slicing(pp))) return BlockShape();
+  double cells = 0;
+  for (int s : slots) cells += static_cast<double>(pp->shots[s].pl->L.nx) * pp->shots[s].pl->L.ny;
+  if (pp->block < 0 && cells > kPoolBlockCells) return BlockShape();
+  const BlockShape bs = block_shape_for(cells, pp->medium_kind);
+  for (int s : slots)
+    if (!block_tiles(pp->shots[s].pl, bs, T)) return BlockShape();
+  return bs;
+}
+
+// An option of the streaming form chooses it.
+void leave_block(fdtd2d_pool *pp) {
+  if (pp->block == 0) return;
+  pp->block = 0;
+  invalidate_lists(pp);
+  pp->graph_valid = false;
+}
 
 bool sliced_cells(const fdtd2d_pool *pp, double cells) { return slicing(pp) && cells >= pp->slice_cells; }
 
@@ -388,6 +457,12 @@ int record_done(fdtd2d_pool *pp) {
 // own kernel on the aux stream beside it.
 int launch_main(fdtd2d_pool *pp, int k) {
   const int gi = pp->ncu * pp->wg_per_cu, gc = pp->ncu * pp->wg_per_cu_cpml;
+  const BlockShape &bs = pp->main_bs;
+  if (bs.C) {
+    const hipError_t eb = fdtd2d::launch_pool_block(pp->d_descs, pp->d_q, k, pp->T, bs.C, bs.R, bs.RG, bs.W, pp->T,
+                                                    pp->medium_kind, block_grid(pp->main_count[0]), pp->stream);
+    return eb == hipSuccess ? FDTD2D_OK : hip_fail(eb, "pool block kernel launch");
+  }
   const bool side = !pp->fused || pp->main_count[2] > 0;
   hipError_t e = hipSuccess;
   if (side) {
@@ -443,7 +518,9 @@ int run_tails(fdtd2d_pool *pp, const std::vector<int> &tails) {
   for (auto &kv : by_t) {
     const int t = kv.first;
     std::vector<int4> lists[fdtd2d::kPoolLists];
-    for (int s : kv.second) append_shot(pp, s, lists);
+    // (tiles made for full launches serve shorter ones)
+    const BlockShape bs = block_shape(pp, kv.second, pp->T);
+    build_lists(pp, kv.second, bs, lists);
     fdtd2d_pool::TailBuf &tb = pp->tailbufs[pp->tail_next];
     pp->tail_next = (pp->tail_next + 1) % fdtd2d_pool::kTailBufs;
     const auto tw = std::chrono::steady_clock::now();
@@ -451,12 +528,16 @@ int run_tails(fdtd2d_pool *pp, const std::vector<int> &tails) {
     pp->blocked_s += seconds_since(tw);
     tb.last_g = pp->g;
     int count[fdtd2d::kPoolLists];
-    int rc = upload_lists(lists, tb.d, tb.cap, count);
+    int rc = upload_lists(lists, bs, tb.d, tb.cap, count);
     if (rc) return rc;
     const int n0 = count[0], n1 = count[1], n2 = count[2];
     const int gi = pp->ncu * pp->wg_per_cu, gc = pp->ncu * pp->wg_per_cu_cpml;
     hipError_t e = fdtd2d::launch_pool_set(pp->d_qt, tb.d, count, pp->g, pp->stream);
-    if (pp->fused) {
+    if (bs.C) {
+      if (e == hipSuccess)
+        e = fdtd2d::launch_pool_block(pp->d_descs, pp->d_qt, 0, pp->T, bs.C, bs.R, bs.RG, bs.W, t, pp->medium_kind, n0,
+                                      pp->stream);
+    } else if (pp->fused) {
       // in stream order: the leftover kernel's tiles are disjoint from the
       // fused kernel's, both read set src and write set 1 - src
       if (e == hipSuccess && n2 > 0)
@@ -682,39 +763,52 @@ int fdtd2d_pool_set_option(fdtd2d_pool *pp, const char *name, double value) {
     if (v < 0) return set_error(FDTD2D_EINVAL, "band must be >= 0");
     pp->band = static_cast<int>(v);
     shape = true;
+    pp->block = 0;  // options of the streaming form choose it
   } else if (n == "band_small" || n == "band_cpml_small") {
     if (v < 0) return set_error(FDTD2D_EINVAL, n + " must be >= 0");
     (n == "band_small" ? pp->band_small : pp->band_cpml_small) = static_cast<int>(v);
     shape = true;
+    pp->block = 0;  // options of the streaming form choose it
   } else if (n == "band_cpml") {
     if (v < 0) return set_error(FDTD2D_EINVAL, "band_cpml must be >= 0");
     pp->band_cpml = static_cast<int>(v);
     shape = true;
+    pp->block = 0;  // options of the streaming form choose it
   } else if (n == "cols_per_lane") {
     if (v != 1 && v != 2) return set_error(FDTD2D_EINVAL, "cols_per_lane must be 1 or 2");
     pp->C = static_cast<int>(v);
     shape = true;
+    pp->block = 0;  // options of the streaming form choose it
   } else if (n == "prefetch") {
     if (v != 1 && v != 2) return set_error(FDTD2D_EINVAL, "prefetch must be 1 or 2");
     pp->D = static_cast<int>(v);
+    leave_block(pp);
     pp->graph_valid = false;
   } else if (n == "fused") {
     if (v != 0 && v != 1) return set_error(FDTD2D_EINVAL, "fused must be 0 or 1");
     pp->fused = static_cast<int>(v);
+    pp->block = 0;
     // the CPML-class entries are routed to lists 1 and 2 by the arrangement
     invalidate_lists(pp);
     pp->graph_valid = false;
   } else if (n == "wg_per_cu") {
     if (v < 1 || v > 8) return set_error(FDTD2D_EINVAL, "wg_per_cu must be 1..8");
     pp->wg_per_cu = static_cast<int>(v);
+    leave_block(pp);
     pp->graph_valid = false;
   } else if (n == "wg_per_cu_cpml") {
     if (v < 1 || v > 8) return set_error(FDTD2D_EINVAL, "wg_per_cu_cpml must be 1..8");
     pp->wg_per_cu_cpml = static_cast<int>(v);
+    leave_block(pp);
     pp->graph_valid = false;
   } else if (n == "graph_chunk") {
     if (v < 0 || v > fdtd2d::kMaxChunk) return set_error(FDTD2D_EINVAL, "graph_chunk must be 0..16");
     pp->chunk = static_cast<int>(v);
+    pp->graph_valid = false;
+  } else if (n == "block") {
+    if (v != 0 && v != 1) return set_error(FDTD2D_EINVAL, "block must be 0 or 1");
+    pp->block = static_cast<int>(v);
+    invalidate_lists(pp);
     pp->graph_valid = false;
   } else if (n == "list_buffers") {
     if (v < 2 || v > fdtd2d_pool::kListBufs) return set_error(FDTD2D_EINVAL, "list_buffers must be 2..4");
@@ -727,6 +821,7 @@ int fdtd2d_pool_set_option(fdtd2d_pool *pp, const char *name, double value) {
     retire(pp, pp->g);
     if (n == "slice_cells") pp->slice_cells = v;
     else pp->slice_every = static_cast<int>(v);
+    invalidate_lists(pp);  // slicing chooses the form
     if (pp->band_small > 0 || pp->band_cpml_small > 0) return reshape(pp);  // a shot's bands follow its class
     for (size_t s = 0; s < pp->shots.size(); ++s)
       if (pp->shots[s].live) fill_desc(pp, static_cast<int>(s));
@@ -759,6 +854,7 @@ int fdtd2d_pool_get_info(const fdtd2d_pool *pp, const char *name, double *value)
   else if (n == "wg_per_cu") *value = pp->wg_per_cu;
   else if (n == "fused") *value = pp->fused;
   else if (n == "wg_per_cu_cpml") *value = pp->wg_per_cu_cpml;
+  else if (n == "block") *value = pp->lists_valid ? pp->main_bs.C > 0 : pp->block != 0;
   else if (n == "graph_chunk") *value = pp->chunk;
   else if (n == "list_buffers") *value = pp->nbufs;
   else if (n == "slice_cells") *value = pp->slice_cells;
