@@ -591,10 +591,10 @@ static std::vector<int4> fused_list(const std::vector<int4> &interior, std::vect
 }
 
 // Measured on MI355X, us per 8-step launch, streaming | {1,4,2,12} |
-// {1,6,3,12} | {2,4,3,12} | {1,8,4,8} (C, R, RG, W):
-//   density  256x192  122 | 12.4 | 16.3 | 16.3 | 18.9    611x1237 121 | 19.3 | 19.8 | 22.5 | 22.2
-//            1024^2   121 | 22.5 | 20.0 | 23.3 | 23.4    1448^2   125 | 35.2 | 33.2 | 32.0 | 35.4
-//            2048^2   123 | 59.4 | 57.7 | 54.1 | 58.4    4096^2   182 |  223 |  207 |  188 |  212
+// {1,6,3,12} | {2,4,4,12} | {1,8,4,8} (C, R, RG, W):
+//   density  256x192  122 | 12.4 | 16.3 | 18.9 | 18.9    611x1237 121 | 18.6 | 20.1 | 24.2 | 22.4
+//            1024^2   120 | 21.6 | 20.2 | 24.1 | 23.1    1448^2   125 | 34.6 | 33.3 | 30.6 | 34.9
+//            2048^2   124 | 59.6 | 57.8 | 52.3 | 58.1    4096^2   182 |  224 |  207 |  182 |  213
 //   table    400^2    206 | 13.3 |    - |    - | 20.6    1024^2   212 | 25.6 |    - |    - | 25.8
 //            2048^2   234 | 68.4 |    - |    - | 64.9    4096^2   323 |  246 |    - |    - |  224
 // Small grids leave the chip idle, so the least work per wave wins; larger
@@ -609,8 +609,8 @@ BlockShape block_shape_for(double cells, int medium_kind) {
 // better one: that moves the state with fewer recomputed cells (four columns
 // in five stored and eleven rows in twelve, against seven in eight and two in
 // three) but its launch lasts as long as its slowest wave, 120 us, so it wins
-// once it fills the chip (density: 2896^2 132 against 95 us, 4096^2 182
-// against 188, 8192^2 638 against 706; table 4096^2 323 against 224).
+// once it fills the chip (density: 2896^2 132 against 90 us, 4096^2 182
+// against 182, 8192^2 638 against 706; table 4096^2 323 against 224).
 static BlockShape pick_block(const fdtd2d_plan *pl) {
   if (pl->block == 0 || pl->pooled) return BlockShape();
   if (pl->block >= 2) return kBlockShapes[pl->block - 2];

@@ -101,7 +101,7 @@ struct BlockShape {
 // The shapes the block kernels are compiled for (block_kernels.hip): the
 // first two for the density medium only (with ca and cb in registers too they
 // would spill).
-constexpr BlockShape kBlockShapes[] = {{2, 4, 3, 12}, {1, 6, 3, 12}, {1, 4, 2, 12}, {1, 8, 4, 8}};
+constexpr BlockShape kBlockShapes[] = {{2, 4, 4, 12}, {1, 6, 3, 12}, {1, 4, 2, 12}, {1, 8, 4, 8}};
 constexpr int kBlockDensityOnly = 2;
 // The shape for grids of `cells` cells in all advanced by one launch.
 BlockShape block_shape_for(double cells, int medium_kind);

@@ -41,15 +41,17 @@ namespace {
 
 constexpr size_t kArenaAlign = 256;
 
-// Cells up to which a launch runs in the block form (block_shape). Measured on
-// MI355X, us per 8-step launch, streaming | block:
-//   density  896^2 shots       4: 329 |  56   16: 343 | 177   32: 442 | 335   64 (51 Mcells): 684 | 650
-//            256..2048 uneven  4: 353 |  78   16: 382 | 272   32: 619 | 578   48 (70 Mcells): 856 | 839
-//            300..600 uneven   4: 313 |  26   16: 339 |  74   64: 367 | 244   (64 of 256..2048, 92 Mcells: 1036 | 1160)
-//   table    896^2 shots       4: 340 |  56   64: 748 | 729   48 of 256..2048: 939 | 934
+// Cells up to which a launch runs in the block form (block_shape), for the
+// table and the density medium. Measured on MI355X, us per 8-step launch,
+// streaming | block:
+//   density  896^2 shots       4: 332 |  48   16: 342 | 160   32: 438 | 298   64 (51 Mcells): 685 | 574
+//            256..2048 uneven  4: 342 |  65   16: 385 | 247   64 (96 Mcells): 1070 | 1028   96 (136): 1443 | 1457
+//                              256 (344 Mcells): 3465 | 3642
+//            300..600 uneven   4: 317 |  27   16: 347 |  59   64: 365 | 194
+//   table    896^2 shots       4: 345 |  58   64: 765 | 737   48 of 256..2048 (70 Mcells): 940 | 937
 // However few its tiles, a streaming launch lasts as long as its slowest wave;
 // with many it keeps every wave busy and recomputes fewer cells.
-constexpr double kPoolBlockCells = 7e7;
+constexpr double kPoolBlockCells[2] = {7e7, 1.1e8};
 
 // First-fit allocator over one device allocation.
 struct Arena {
@@ -355,7 +357,7 @@ BlockShape block_shape(const fdtd2d_pool *pp, const std::vector<int> &slots, int
   if (pp->block == 0 || slots.empty() || (pp->block < 0 && slicing(pp))) return BlockShape();
   double cells = 0;
   for (int s : slots) cells += static_cast<double>(pp->shots[s].pl->L.nx) * pp->shots[s].pl->L.ny;
-  if (pp->block < 0 && cells > kPoolBlockCells) return BlockShape();
+  if (pp->block < 0 && cells > kPoolBlockCells[pp->medium_kind == FDTD2D_MEDIUM_DENSITY]) return BlockShape();
   const BlockShape bs = block_shape_for(cells, pp->medium_kind);
   for (int s : slots)
     if (!block_tiles(pp->shots[s].pl, bs, T)) return BlockShape();

@@ -428,10 +428,9 @@ int fdtd2d_plan_kernel_time(fdtd2d_plan *plan, int cls, double *avg_ms, int *cou
  * "wg_per_cu_cpml" (persistent work-groups per CU of the interior or fused
  * kernel / of the CPML-class kernel, default 3 / 2), "block" (0 or 1: the
  * form that keeps a tile in registers for a whole launch off or on; by default
- * on for launches of up to 70 million cells without time slicing, and off from
- * the first option above but "tblock" on, which belong to the other form),
- * "graph_chunk" (0..16,
- * 0 = no graphs), "list_buffers" (2..4, default 4: device copies of the
+ * on for launches of up to 110 million cells (table medium: 70 million)
+ * without time slicing, and off from the first option above but "tblock" on,
+ * which belong to the other form), "graph_chunk" (0..16, 0 = no graphs), "list_buffers" (2..4, default 4: device copies of the
  * tile lists, each kept for the shot set it holds; a rebuild of the lists
  * waits for the launches that read the copy it reuses), "slice_cells" and
  * "slice_every" (time slicing, default off: shots of at least slice_cells
