@@ -14,21 +14,35 @@ namespace {
 // stays; the scan (j from ny-3 down while |Ez| < edge) stops at the largest
 // j >= 1 whose |Ez| is not below the edge, else at 0. Only the edge level
 // carries from step to step: two waves per step find the launch's maxima side
-// by side, one thread runs the edge through them, the waves scan. (Step by
-// step, two block reductions each, a line took 79 us per 8-step launch at
-// 3000 rows, all of it latency, after a step kernel of 45; now 14.6.)
+// by side, one thread runs the edge through them, the waves scan. A wave has
+// the first kAhead rows of its scan, and of its maximum, in flight together
+// (clamped rows repeat one that counts anyway): the kernel is latency, 21
+// work-groups. (Step by step, two block reductions each, a line took 79 us per
+// 8-step launch at 3000 rows behind a step kernel of 40; side by side with
+// eight loads in flight 14.6; now 7.1.)
 __global__ void __launch_bounds__(128 * kMaxT) rc_kernel(const RcArgs r, int n0, int t) {
+  constexpr int kAhead = 24;  // 3072 rows
   __shared__ float s_max[kMaxT][2], s_first[kMaxT], s_edge[kMaxT];
   __shared__ int s_j[kMaxT][2];
   const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, half = (tid >> 6) & 1, s = tid >> 7;
-  const int ny = r.ny;
-  const int ncand = 1 + max(0, (ny - 2) - r.jcut);
+  const int ny = r.ny, at = half * 64 + lane;
+  const int ncand = 1 + max(0, (ny - 2) - r.jcut), last = ny - 3;  // rows 1 .. last are scanned
   const long long slot = (n0 + s) & (kMaxT - 1);
+  const float *cm = r.cap + (slot * r.nprobe + r.map[2 * e]) * ny;
+  const float *cs = r.cap + (slot * r.nprobe + r.map[2 * e + 1]) * ny;
+  float scan[kAhead];
   if (s < t) {
-    const float *cm = r.cap + (slot * r.nprobe + r.map[2 * e]) * ny;
+    auto cand = [&](int q) { return q <= 0 ? cm[0] : cm[r.jcut + min(q, ncand - 1) - 1]; };
+    float v[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      v[k] = cand(ncand == 1 ? 0 : at + 128 * k);
+      scan[k] = cs[max(0, min(1 + at + 128 * k, last))];
+    }
     float m = -INFINITY;
-#pragma unroll 8
-    for (int q = half * 64 + lane; q < ncand; q += 128) m = fmaxf(m, q == 0 ? cm[0] : cm[r.jcut + q - 1]);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) m = fmaxf(m, v[k]);
+    for (int q = at + 128 * kAhead; q < ncand; q += 128) m = fmaxf(m, cand(q));
     for (int w = 32; w > 0; w >>= 1) m = fmaxf(m, __shfl_xor(m, w));
     if (lane == 0) {
       s_max[s][half] = m;
@@ -48,12 +62,15 @@ __global__ void __launch_bounds__(128 * kMaxT) rc_kernel(const RcArgs r, int n0,
   }
   __syncthreads();
   if (s < t) {
-    const float *cs = r.cap + (slot * r.nprobe + r.map[2 * e + 1]) * ny;
     const float edge = s_edge[s];
     int bj = 0;
-#pragma unroll 8
-    for (int j = 1 + half * 64 + lane; j <= ny - 3; j += 128)
-      if (!(fabsf(cs[j]) < edge)) bj = j;  // j grows: the last one is the largest
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int j = 1 + at + 128 * k;
+      if (j <= last && !(fabsf(scan[k]) < edge)) bj = j;  // j grows: the last one is the largest
+    }
+    for (int j = 1 + at + 128 * kAhead; j <= last; j += 128)
+      if (!(fabsf(cs[j]) < edge)) bj = j;
     for (int w = 32; w > 0; w >>= 1) bj = max(bj, __shfl_xor(bj, w));
     if (lane == 0) s_j[s][half] = bj;
   }

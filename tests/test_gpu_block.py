@@ -120,7 +120,7 @@ def test_default_form_and_options(gpu_device):
         assert np.array_equal(_bits(want[k]), _bits(got[k])), k
 
 
-@pytest.mark.parametrize("ny", [66, 133, 300])
+@pytest.mark.parametrize("ny", [66, 133, 300, 3300])
 @pytest.mark.parametrize("jcut", [0, 9, 64, 500])
 def test_rc_candidates(gpu_device, ny, jcut):
     """The RC maximum over row 0 and rows jcut .. ny-3 (none past the grid),
