@@ -8,22 +8,21 @@ namespace fdtd2d {
 namespace {
 
 // Calls f with the shape as constants: C, R, RG, W, the medium, and the waves
-// per SIMD the registers are held to: two work-groups per CU. (Only waves with
-// events spill for it, 18 registers at four rows each.)
+// per SIMD the registers are held to: two work-groups per CU. (For it only
+// waves with events spill, up to 20 registers.)
 template <class F>
 hipError_t with_shape(int C, int R, int RG, int W, int medium_kind, F f) {
   const int key = ((C * 16 + R) * 16 + RG) * 16 + W;
   constexpr auto k = [](int c, int r, int rg, int w) { return ((c * 16 + r) * 16 + rg) * 16 + w; };
   const bool table = medium_kind == kTable;
   if (key == k(2, 4, 4, 12) && !table) return f.template operator()<2, 4, 4, 12, kDensity, 6>();
-  if (key == k(1, 6, 3, 12) && !table) return f.template operator()<1, 6, 3, 12, kDensity, 6>();
+  if (key == k(1, 6, 3, 12)) {
+    if (table) return f.template operator()<1, 6, 3, 12, kTable, 6>();
+    return f.template operator()<1, 6, 3, 12, kDensity, 6>();
+  }
   if (key == k(1, 4, 2, 12)) {
     if (table) return f.template operator()<1, 4, 2, 12, kTable, 6>();
     return f.template operator()<1, 4, 2, 12, kDensity, 6>();
-  }
-  if (key == k(1, 8, 4, 8)) {
-    if (table) return f.template operator()<1, 8, 4, 8, kTable, 4>();
-    return f.template operator()<1, 8, 4, 8, kDensity, 4>();
   }
   return hipErrorInvalidValue;
 }

@@ -591,18 +591,19 @@ static std::vector<int4> fused_list(const std::vector<int4> &interior, std::vect
 }
 
 // Measured on MI355X, us per 8-step launch, streaming | {1,4,2,12} |
-// {1,6,3,12} | {2,4,4,12} | {1,8,4,8} (C, R, RG, W):
-//   density  256x192  122 | 12.4 | 16.3 | 18.9 | 18.9    611x1237 121 | 18.6 | 20.1 | 24.2 | 22.4
-//            1024^2   120 | 21.6 | 20.2 | 24.1 | 23.1    1448^2   125 | 34.6 | 33.3 | 30.6 | 34.9
-//            2048^2   124 | 59.6 | 57.8 | 52.3 | 58.1    4096^2   182 |  224 |  207 |  182 |  213
-//   table    400^2    206 | 13.3 |    - |    - | 20.6    1024^2   212 | 25.6 |    - |    - | 25.8
-//            2048^2   234 | 68.4 |    - |    - | 64.9    4096^2   323 |  246 |    - |    - |  224
+// {1,6,3,12} | {2,4,4,12} (C, R, RG, W):
+//   density  256x192  122 | 12.4 | 16.3 | 18.9    611x1237 121 | 18.6 | 20.1 | 24.2
+//            1024^2   120 | 21.6 | 20.2 | 24.1    1448^2   125 | 34.6 | 33.3 | 30.6
+//            2048^2   124 | 59.6 | 57.8 | 52.3    4096^2   182 |  224 |  207 |  182
+//   table    400^2    206 | 13.3 | 16.9           700x900  209 | 20.0 | 24.1
+//            1024^2   212 | 25.2 | 24.6           500x3000 217 | 43.1 | 36.9
+//            2048^2   234 | 68.5 | 63.5           4096^2   323 |  248 |  215
 // Small grids leave the chip idle, so the least work per wave wins; larger
 // ones fill it, and the fewest recomputed cells win (more rows per wave, then
 // two columns per lane).
 BlockShape block_shape_for(double cells, int medium_kind) {
-  if (medium_kind == FDTD2D_MEDIUM_TABLE) return kBlockShapes[cells < 1.1e6 ? 2 : 3];
-  return kBlockShapes[cells < 7.5e5 ? 2 : cells < 1.5e6 ? 1 : 0];
+  if (cells < (medium_kind == FDTD2D_MEDIUM_TABLE ? 9e5 : 7.5e5)) return kBlockShapes[2];
+  return kBlockShapes[medium_kind == FDTD2D_MEDIUM_TABLE || cells < 1.3e6 ? 1 : 0];
 }
 
 // The block form's shape for a plan, or none where the streaming form is the
@@ -610,7 +611,7 @@ BlockShape block_shape_for(double cells, int medium_kind) {
 // in five stored and eleven rows in twelve, against seven in eight and two in
 // three) but its launch lasts as long as its slowest wave, 120 us, so it wins
 // once it fills the chip (density: 2896^2 132 against 90 us, 4096^2 182
-// against 182, 8192^2 638 against 706; table 4096^2 323 against 224).
+// against 182, 8192^2 638 against 706; table 4096^2 323 against 215).
 static BlockShape pick_block(const fdtd2d_plan *pl) {
   if (pl->block == 0 || pl->pooled) return BlockShape();
   if (pl->block >= 2) return kBlockShapes[pl->block - 2];
@@ -1442,7 +1443,7 @@ int fdtd2d_plan_set_option(fdtd2d_plan *pl, const char *name, double value) {
   } else if (n == "block") {
     if (v < 0 || v > 1 + static_cast<int>(std::size(kBlockShapes)) ||
         (v >= 2 && v - 2 < kBlockDensityOnly && pl->a.medium_kind == FDTD2D_MEDIUM_TABLE))
-      return set_error(FDTD2D_EINVAL, "block must be 0 (off), 1 (on) or 2 .. 5 (a shape; table medium: 4 or 5)");
+      return set_error(FDTD2D_EINVAL, "block must be 0 (off), 1 (on) or 2 .. 4 (a shape; table medium: 3 or 4)");
     pl->block = v;
   } else if (n == "prefetch") {
     const int maxd = pl->C == 1 ? 4 : pl->C == 2 ? 2 : 1;

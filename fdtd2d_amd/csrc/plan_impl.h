@@ -99,10 +99,10 @@ struct BlockShape {
   bool operator==(const BlockShape &o) const { return C == o.C && R == o.R && RG == o.RG && W == o.W; }
 };
 // The shapes the block kernels are compiled for (block_kernels.hip): the
-// first two for the density medium only (with ca and cb in registers too they
-// would spill).
-constexpr BlockShape kBlockShapes[] = {{2, 4, 4, 12}, {1, 6, 3, 12}, {1, 4, 2, 12}, {1, 8, 4, 8}};
-constexpr int kBlockDensityOnly = 2;
+// first for the density medium only (with ca and cb in registers too it would
+// spill).
+constexpr BlockShape kBlockShapes[] = {{2, 4, 4, 12}, {1, 6, 3, 12}, {1, 4, 2, 12}};
+constexpr int kBlockDensityOnly = 1;
 // The shape for grids of `cells` cells in all advanced by one launch.
 BlockShape block_shape_for(double cells, int medium_kind);
 bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMasks *m,

@@ -48,10 +48,10 @@ constexpr size_t kArenaAlign = 256;
 //            256..2048 uneven  4: 342 |  65   16: 385 | 247   64 (96 Mcells): 1070 | 1028   96 (136): 1443 | 1457
 //                              256 (344 Mcells): 3465 | 3642
 //            300..600 uneven   4: 317 |  27   16: 347 |  59   64: 365 | 194
-//   table    896^2 shots       4: 345 |  58   64: 765 | 737   48 of 256..2048 (70 Mcells): 940 | 937
+//   table    896^2 shots       4: 340 |  53   64: 766 | 657   256..2048 uneven  64 (96 Mcells): 1206 | 1213
 // However few its tiles, a streaming launch lasts as long as its slowest wave;
 // with many it keeps every wave busy and recomputes fewer cells.
-constexpr double kPoolBlockCells[2] = {7e7, 1.1e8};
+constexpr double kPoolBlockCells[2] = {9e7, 1.1e8};
 
 // First-fit allocator over one device allocation.
 struct Arena {

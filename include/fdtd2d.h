@@ -325,9 +325,10 @@ int fdtd2d_plan_set_tblock(fdtd2d_plan *plan, int steps_per_launch);
    the grid has them; 0: all CPML-class tiles in the second kernel; with 4
    columns per lane launches are never fused), "block" (the form that keeps a
    tile in registers for a whole launch: 0 off, 1 on, 2 .. 4 on with a given
-   shape; by default on for grids up to about 3400^2 cells (table medium:
-   4900^2) unless a wave would hold more than 64 events; the options above
-   but "tblock" belong to the other form and switch this one off). Results
+   shape, the table medium 3 or 4; by default on for grids up to 15 million
+   cells, table medium 24 million, unless a wave would hold more than 64
+   events; the options above but "tblock" belong to the other form and switch
+   this one off). Results
    are identical for every choice. */
 int fdtd2d_plan_set_option(fdtd2d_plan *plan, const char *name, double value);
 /* Plan facts by name: "pitch", "tblock", "band", "band_cpml", "ntx", "nty",
@@ -428,7 +429,7 @@ int fdtd2d_plan_kernel_time(fdtd2d_plan *plan, int cls, double *avg_ms, int *cou
  * "wg_per_cu_cpml" (persistent work-groups per CU of the interior or fused
  * kernel / of the CPML-class kernel, default 3 / 2), "block" (0 or 1: the
  * form that keeps a tile in registers for a whole launch off or on; by default
- * on for launches of up to 110 million cells (table medium: 70 million)
+ * on for launches of up to 110 million cells (table medium: 90 million)
  * without time slicing, and off from the first option above but "tblock" on,
  * which belong to the other form), "graph_chunk" (0..16, 0 = no graphs), "list_buffers" (2..4, default 4: device copies of the
  * tile lists, each kept for the shot set it holds; a rebuild of the lists

@@ -17,7 +17,7 @@ from helpers import all_state, random_problem
 pytestmark = pytest.mark.gpu
 
 # "block" option: the compiled shapes of each medium
-SHAPES = {False: [2, 3, 4, 5], True: [4, 5]}
+SHAPES = {False: [2, 3, 4], True: [3, 4]}
 
 
 def _bits(a):
