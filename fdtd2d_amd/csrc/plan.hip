@@ -607,9 +607,9 @@ BlockShape block_shape_for(double cells, int medium_kind) {
 }
 
 // The block form's shape for a plan, or none where the streaming form is the
-// better one: that moves the state with fewer recomputed cells (four columns
-// in five stored and eleven rows in twelve, against seven in eight and two in
-// three) but its launch lasts as long as its slowest wave, 120 us, so it wins
+// better one: that moves the state with fewer recomputed cells (it stores
+// 96 of about 112 rows it steps, the block form 32 of 48; columns are 112 of
+// 128 in both) but its launch lasts as long as its slowest wave, 120 us, so it wins
 // once it fills the chip (density: 2896^2 132 against 90 us, 4096^2 182
 // against 182, 8192^2 638 against 706; table 4096^2 323 against 215).
 static BlockShape pick_block(const fdtd2d_plan *pl) {
@@ -710,6 +710,11 @@ int set_tiling(fdtd2d_plan *pl) {
   BlockShape bs = pick_block(pl);
   std::vector<fdtd2d::BlockTile> blocks;
   if (bs.C && !make_blocks(pl->L.nx, pl->L.ny, pl->a.P, T, bs, &m, blocks)) bs = BlockShape();
+  // (a long narrow grid's block tiles can take more than the static array
+  // holds; its streaming tiles may not)
+  if (pl->static_lists && blocks.size() * sizeof(fdtd2d::BlockTile) > kStaticListEntries * sizeof(int4))
+    bs = BlockShape();
+  if (!bs.C) blocks.clear();
   if (bs.C) {
     lists[1].clear();
     lists[0].resize(blocks.size() * (sizeof(fdtd2d::BlockTile) / sizeof(int4)));

@@ -13,6 +13,7 @@ import fdtd2d_amd as F
 from oracle.oracle import Oracle
 
 from helpers import all_state, random_problem
+from test_zz_no_alloc import _DeviceBuffer
 
 pytestmark = pytest.mark.gpu
 
@@ -118,6 +119,25 @@ def test_default_form_and_options(gpu_device):
             plan.set_option("block", 9)
     for k in want:
         assert np.array_equal(_bits(want[k]), _bits(got[k])), k
+
+
+def test_static_lists_limit(gpu_device):
+    """A plan in the caller's memory on a long narrow grid, whose smallest
+    block tiles (about 23000 of 48 bytes) exceed the 1 MiB static list array,
+    keeps the streaming form; a small grid's run from that array."""
+    for nx, ny, block in ((130, 250000, 0), (200, 180, 1)):
+        box = F.Setup.box(nx, ny, 4, 4, 1e-3)
+        need = box.footprint()
+        buf = _DeviceBuffer(need)
+        plan = F.Plan.in_memory(box, gpu_device, buf.ptr, need)
+        try:
+            plan.set_option("block", 4)
+            assert plan.info("block") == block
+            plan.run(4)
+            plan.sync()
+        finally:
+            plan.close()
+            buf.free()
 
 
 @pytest.mark.parametrize("ny", [66, 133, 300, 3300])
