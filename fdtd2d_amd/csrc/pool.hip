@@ -7,7 +7,9 @@
 // The shots' tile entries are concatenated into two packed lists (interior,
 // CPML class), one work-group of 4 entries per shot at a time, and two
 // persistent kernels (one per class, on two streams) drain them through a
-// ticket queue in device memory. Per-shot parameters live in a descriptor
+// ticket queue in device memory. Up to 90 (table) or 110 (density) million
+// cells per launch the shots run in the block form instead (block_device.h):
+// one list of block tiles and one kernel, a work-group per tile. Per-shot parameters live in a descriptor
 // table; a shot's step index and buffer set follow from the pool's launch
 // counter g, which a one-wave tick kernel advances on the device. Nothing a
 // launch reads changes its address, so a chunk of launches can be captured
