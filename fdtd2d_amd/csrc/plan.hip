@@ -807,10 +807,28 @@ static void plasma_runs(const fdtd2d_problem *p, fdtd2d_plan *pl) {
 // A 2D copy moves one row at a time, 7-10 us each (1024^2: 6.9 ms, 8192^2: 82
 // ms, 500x3000: 22 ms); a contiguous one runs at the link's rate (4 MB in 0.2
 // ms, 268 MB in 25 ms). So rows that are contiguous on the device go in one
-// copy, and others pass a packed device buffer, at most kPackBytes of rows at
-// a time, allocated for the call (a plan made by fdtd2d_plan_create_in, which
-// allocates nothing, and a device without that much left keep the 2D copy).
-constexpr size_t kPackBytes = size_t{64} << 20;
+// copy, and others pass the plan's packing buffer, as many rows at a time as
+// it holds. The buffer is kept: hipFree waits for all work on the device, and
+// a read must not wait for launches of other plans or shots (a finished shot
+// read beside 0.6 s of queued launches took 240 ms with a buffer freed in the
+// call). A plan made by fdtd2d_plan_create_in, which allocates nothing, a
+// device without that much left and rows longer than the buffer take the 2D
+// copy.
+static float *pack_buffer(fdtd2d_plan *pl, size_t row) {
+  if (pl->static_lists) return nullptr;
+  PackBuffer &b = *pl->pack;
+  if (!b.d) {
+    // a plan's own: no more than its largest field
+    const size_t need = pl->pooled ? kPackBytes : std::min(kPackBytes, static_cast<size_t>(pl->L.ny) * pl->L.nx * 4);
+    if (hipMalloc(reinterpret_cast<void **>(&b.d), need) != hipSuccess) {
+      (void)hipGetLastError();
+      b.d = nullptr;
+      return nullptr;
+    }
+    b.bytes = need;
+  }
+  return row <= b.bytes ? b.d : nullptr;
+}
 
 // rows x cols floats between packed (row length cols) and one or two pitched
 // planes; to_plane: from packed into them.
@@ -844,12 +862,7 @@ static int copy_rows(fdtd2d_plan *pl, float *d0, float *d1, size_t pitch, int ro
     return FDTD2D_OK;
   }
   const size_t row = static_cast<size_t>(cols) * 4;
-  const int slab = static_cast<int>(std::min<size_t>(rows, std::max<size_t>(1, kPackBytes / row)));
-  float *tmp = nullptr;
-  if (rows > 1 && !pl->static_lists && hipMalloc(reinterpret_cast<void **>(&tmp), slab * row) != hipSuccess) {
-    (void)hipGetLastError();
-    tmp = nullptr;
-  }
+  float *tmp = rows > 1 ? pack_buffer(pl, row) : nullptr;
   if (!tmp) {
     if (out)
       HIP_TRY(hipMemcpy2D(out, row, d0, pitch * 4, row, rows, hipMemcpyDeviceToHost), "hipMemcpy2D D2H rows");
@@ -858,6 +871,7 @@ static int copy_rows(fdtd2d_plan *pl, float *d0, float *d1, size_t pitch, int ro
         if (d) HIP_TRY(hipMemcpy2D(d, pitch * 4, in, row, row, rows, hipMemcpyHostToDevice), "hipMemcpy2D H2D rows");
     return FDTD2D_OK;
   }
+  const int slab = static_cast<int>(std::min<size_t>(rows, pl->pack->bytes / row));
   hipError_t e = hipSuccess;
   for (int r = 0; r < rows && e == hipSuccess; r += slab) {
     const int n = std::min(slab, rows - r);
@@ -871,7 +885,6 @@ static int copy_rows(fdtd2d_plan *pl, float *d0, float *d1, size_t pitch, int ro
     if (e == hipSuccess) e = hipStreamSynchronize(pl->stream);
     if (e == hipSuccess && out) e = hipMemcpy(out + at, tmp, n * row, hipMemcpyDeviceToHost);
   }
-  hipFree(tmp);
   if (e != hipSuccess) return hip_fail(e, "copying rows");
   return FDTD2D_OK;
 }
@@ -1756,6 +1769,7 @@ int fdtd2d_plan_destroy(fdtd2d_plan *pl) {
   } else if (pl->wg_buf && !pl->static_lists) {
     hipFree(pl->wg_buf);
   }
+  if (pl->own_pack.d) hipFree(pl->own_pack.d);
   if (pl->base && pl->owns_base) hipFree(pl->base);
   if (pl->aux) hipStreamDestroy(pl->aux);
   if (pl->own_stream) hipStreamDestroy(pl->own_stream);

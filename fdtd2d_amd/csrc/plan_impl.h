@@ -108,6 +108,15 @@ BlockShape block_shape_for(double cells, int medium_kind);
 bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMasks *m,
                  std::vector<fdtd2d::BlockTile> &out);
 
+// Device rows packed for a copy to or from the host (copy_rows), allocated at
+// the first copy that needs it, kept and freed by its owner: a plan, or a pool
+// for all of its shots.
+constexpr size_t kPackBytes = size_t{16} << 20;
+struct PackBuffer {
+  float *d = nullptr;
+  size_t bytes = 0;
+};
+
 Layout make_layout(const fdtd2d_problem *p, size_t n_events);
 int hip_fail(hipError_t e, const char *what);
 
@@ -128,6 +137,7 @@ struct fdtd2d_plan {
   char *base = nullptr;
   fdtd2d::detail::Layout L{};
   fdtd2d::StepArgs a{};
+  fdtd2d::detail::PackBuffer own_pack, *pack = &own_pack;  // pooled: the pool's
   int src = 0;
   int n = 0;
   int nsteps = 0;

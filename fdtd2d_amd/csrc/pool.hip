@@ -154,6 +154,7 @@ struct fdtd2d_pool {
   // memory
   size_t budget = 0;
   Arena arena;
+  PackBuffer pack;  // the shots' reads (outside the budget, as the lists are)
   // shots
   std::vector<Shot> shots;
   std::vector<int> free_slots;
@@ -942,6 +943,7 @@ int fdtd2d_pool_add(fdtd2d_pool *pp, const fdtd2d_problem *p, int *shot) {
   Shot &sh = pp->shots[slot];
   sh = Shot();
   sh.pl = pl;
+  pl->pack = &pp->pack;
   sh.live = true;
   sh.bytes = bytes;
   sh.medium_kind = p->medium_kind;
@@ -1063,6 +1065,7 @@ int fdtd2d_pool_destroy(fdtd2d_pool *pp) {
   if (pp->d_q) hipFree(pp->d_q);
   if (pp->d_qt) hipFree(pp->d_qt);
   if (pp->arena.base) hipFree(pp->arena.base);
+  if (pp->pack.d) hipFree(pp->pack.d);
   if (pp->ev_fork) hipEventDestroy(pp->ev_fork);
   if (pp->ev_join) hipEventDestroy(pp->ev_join);
   if (pp->aux) hipStreamDestroy(pp->aux);
