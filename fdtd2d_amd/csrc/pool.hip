@@ -596,31 +596,52 @@ int reshape(fdtd2d_pool *pp) {
   return FDTD2D_OK;
 }
 
+// The shots of the next launch: those with a full launch's steps left and the
+// tails; sliced shots sit out the launches between their turns.
+struct NextLaunch {
+  std::vector<int> main_set, tails;
+  int min_left = 1 << 30;   // steps left, least of main_set
+  bool any_sliced = false;  // sliced shots run, at this turn or another
+};
+
+NextLaunch next_launch(const fdtd2d_pool *pp) {
+  NextLaunch l;
+  const bool slice_turn = pp->g % std::max(pp->slice_every, 1) == 0;
+  for (size_t s = 0; s < pp->shots.size(); ++s) {
+    const Shot &sh = pp->shots[s];
+    if (!sh.live || sh.finished) continue;
+    if (sliced(pp, sh.pl)) {
+      l.any_sliced = true;
+      if (!slice_turn) continue;
+    }
+    const int left = sh.pl->nsteps - sh.pl->n;
+    if (left >= pp->T) {
+      l.main_set.push_back(static_cast<int>(s));
+      l.min_left = std::min(l.min_left, left);
+    } else {
+      l.tails.push_back(static_cast<int>(s));
+    }
+  }
+  return l;
+}
+
+// Whether the next launch runs in the block form (the tails taken together
+// where it has only those); with no shot to run, whether the options allow it.
+bool next_in_block_form(const fdtd2d_pool *pp) {
+  const NextLaunch l = next_launch(pp);
+  const std::vector<int> &set = l.main_set.empty() ? l.tails : l.main_set;
+  if (set.empty()) return pp->block > 0 || (pp->block < 0 && !slicing(pp));
+  if (pp->lists_valid && set == pp->main_set) return pp->main_bs.C > 0;
+  return block_shape(pp, set, pp->T).C > 0;
+}
+
 int step_impl(fdtd2d_pool *pp, int nlaunch) {
   HIP_TRY(hipSetDevice(pp->device), "hipSetDevice");
   while (nlaunch > 0) {
-    std::vector<int> main_set, tails;
-    int min_left = 1 << 30;
-    // time slicing: sliced shots sit out the launches between their turns
-    const bool slice_turn = pp->g % std::max(pp->slice_every, 1) == 0;
-    bool any_sliced = false;
-    for (size_t s = 0; s < pp->shots.size(); ++s) {
-      const Shot &sh = pp->shots[s];
-      if (!sh.live || sh.finished) continue;
-      if (sliced(pp, sh.pl)) {
-        any_sliced = true;
-        if (!slice_turn) continue;
-      }
-      const int left = sh.pl->nsteps - sh.pl->n;
-      if (left >= pp->T) {
-        main_set.push_back(static_cast<int>(s));
-        min_left = std::min(min_left, left);
-      } else {
-        tails.push_back(static_cast<int>(s));
-      }
-    }
+    const NextLaunch next = next_launch(pp);
+    const std::vector<int> &main_set = next.main_set, &tails = next.tails;
     if (main_set.empty() && tails.empty()) {
-      if (!any_sliced) break;
+      if (!next.any_sliced) break;
       // only sliced shots run and this is not their turn: move the launch
       // counter (host and device) on to their next turn, launching nothing
       const int skip = fdtd2d::policy::to_next_turn(pp->g, pp->slice_every);
@@ -634,7 +655,7 @@ int step_impl(fdtd2d_pool *pp, int nlaunch) {
       if (rc) return rc;
     }
     const bool use_graph = pp->chunk > 0 && nlaunch >= pp->chunk && tails.empty() && !main_set.empty() &&
-                           min_left >= pp->chunk * pp->T && !any_sliced;
+                           next.min_left >= pp->chunk * pp->T && !next.any_sliced;
     if (use_graph) {
       if (!pp->graph_valid) {
         int rc = capture_graph(pp);
@@ -859,7 +880,7 @@ int fdtd2d_pool_get_info(const fdtd2d_pool *pp, const char *name, double *value)
   else if (n == "wg_per_cu") *value = pp->wg_per_cu;
   else if (n == "fused") *value = pp->fused;
   else if (n == "wg_per_cu_cpml") *value = pp->wg_per_cu_cpml;
-  else if (n == "block") *value = pp->lists_valid ? pp->main_bs.C > 0 : pp->block != 0;
+  else if (n == "block") *value = next_in_block_form(pp);
   else if (n == "graph_chunk") *value = pp->chunk;
   else if (n == "list_buffers") *value = pp->nbufs;
   else if (n == "slice_cells") *value = pp->slice_cells;
