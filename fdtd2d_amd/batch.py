@@ -16,8 +16,9 @@ from __future__ import annotations
 import time
 from concurrent.futures import ThreadPoolExecutor
 
+from ._lib import MEDIUM_TABLE
 from .problem import Pool, Setup
-from .tuning import ShapeCache, mix_key
+from .tuning import ShapeCache, form_key, mix_key
 
 # coordinate-descent axes, in the order they are tuned; the first value of
 # each is the starting point (the shape that won on uneven shot mixes)
@@ -126,6 +127,15 @@ def shot_sizes(setups):
     return out
 
 
+def pool_key(pool, sizes) -> str:
+    """Key of a mix of `sizes` (shot_sizes) for a pool that is to hold them
+    all, in the form their launches will take."""
+    key = mix_key(sizes)
+    limit = pool.info("block_cells_table" if any(z[3] == MEDIUM_TABLE for z in sizes) else "block_cells_density")
+    cells = sum(float(nx) * ny for nx, ny, _, _ in sizes)
+    return form_key(key, cells <= limit and pool.info("block") > 0)
+
+
 def cached_shape(pool, key: str, cache: ShapeCache | None, log=None) -> dict | None:
     """Sets the shape cached for the mix `key` on the pool (best before its
     shots are added: a shape change retiles every shot) and returns its
@@ -144,9 +154,10 @@ def cached_shape(pool, key: str, cache: ShapeCache | None, log=None) -> dict | N
 
 def choose_shape(pool, key: str, cache: ShapeCache | None, log=None, lookup: bool = True) -> dict:
     """The launch shape for the shots now in the pool: the cached one for
-    their mix when there is one (no trials; lookup=False skips the cache),
-    else the autotuner's, which is then stored. Returns the autotune record
-    with "source" (the cache file or "trials") and "key"."""
+    their mix and form (form_key) when there is one (no trials; lookup=False
+    skips the cache), else the autotuner's, which is then stored. Returns the
+    autotune record with "source" (the cache file or "trials") and "key"."""
+    key = form_key(key, _block_form(pool))
     hit = cached_shape(pool, key, cache, log) if lookup else None
     if hit is not None:
         return hit
@@ -180,7 +191,7 @@ def run_pool(setups, device: int = 0, tune: bool = True, chunk_launches: int = 8
     time in stats["seconds"] runs from the shots being resident to the last
     launch's end, trials included."""
     pool = Pool(device, **options)
-    key = mix_key(shot_sizes(setups))
+    key = pool_key(pool, shot_sizes(setups))
     tuned = cached_shape(pool, key, cache, log) if tune and lookup else None
     if warmup and tuned is not None and setups:
         warm_up(setups[0], device, tuned["shape"], **options)

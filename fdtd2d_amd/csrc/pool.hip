@@ -881,6 +881,8 @@ int fdtd2d_pool_get_info(const fdtd2d_pool *pp, const char *name, double *value)
   else if (n == "fused") *value = pp->fused;
   else if (n == "wg_per_cu_cpml") *value = pp->wg_per_cu_cpml;
   else if (n == "block") *value = next_in_block_form(pp);
+  else if (n == "block_cells_table") *value = kPoolBlockCells[0];
+  else if (n == "block_cells_density") *value = kPoolBlockCells[1];
   else if (n == "graph_chunk") *value = pp->chunk;
   else if (n == "list_buffers") *value = pp->nbufs;
   else if (n == "slice_cells") *value = pp->slice_cells;

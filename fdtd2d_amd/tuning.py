@@ -14,6 +14,12 @@ entry of the same medium and device whose bucket shares are closest (L1
 distance at most ``max_distance`` tenths), for streams whose mix is only
 known from a sample.
 
+Pools and plans that run in the block form (by their total cells, which a key's
+shares do not tell) have keys of their own (form_key): a streaming shape tuned
+on many cells would switch that form off where it is several times faster, and
+{"block": 1} from few would force it on where it loses. Such a shape under any
+other key is passed over.
+
 Single plans are keyed the same way by their own grid (plan_key: the size
 bucket of each side, the CPML thickness and the medium), under kind "plan";
 tune_plan finds a plan's shape by coordinate descent on the live plan.
@@ -61,6 +67,18 @@ def mix_key(shots) -> str:
     return "m" + "+".join(str(m) for m in sorted(media)) + "|" + ",".join(parts)
 
 
+def form_key(key: str, block: bool) -> str:
+    """The key of the same mix or grid for a pool or plan that runs in the
+    block form, or in the streaming form."""
+    media, bar, rest = key.partition("|")
+    media = media.removesuffix("b")
+    return (media + "b" if block and media else media) + bar + rest
+
+
+def is_block_key(key: str) -> bool:
+    return key.partition("|")[0].endswith("b")
+
+
 def _shares(key: str):
     media, _, parts = key.partition("|")
     return media, {int(p.split(":")[0]): int(p.split(":")[1]) for p in parts.split(",") if p}
@@ -68,7 +86,7 @@ def _shares(key: str):
 
 def key_distance(a: str, b: str) -> float:
     """L1 distance between the bucket shares of two keys (tenths); infinite
-    across media."""
+    across media and forms."""
     ma, sa = _shares(a)
     mb, sb = _shares(b)
     if ma != mb:
@@ -102,6 +120,8 @@ class ShapeCache:
         for src, entries in self._sources():
             for e in entries:
                 if e.get("kind") != kind or int(e.get("cus", -1)) != int(cus):
+                    continue
+                if isinstance(e["shape"], dict) and e["shape"].get("block") and not is_block_key(e["key"]):
                     continue
                 if e["key"] == key:
                     return dict(e["shape"]), src
@@ -162,6 +182,13 @@ def _plan_trial(plan, launches: int) -> float:
     return float(plan.nx) * plan.ny * steps / dt if dt > 0 else 0.0
 
 
+def _block_form(plan) -> bool:
+    try:
+        return plan.info("block") > 0
+    except (KeyError, FDTD2DError):
+        return False
+
+
 def tune_plan(plan, launches: int = 4, axes=PLAN_AXES, log=None) -> dict:
     """Coordinate descent over the plan's launch shape (columns per lane,
     band rows, prefetch depth) on the live plan: every trial advances the
@@ -172,10 +199,7 @@ def tune_plan(plan, launches: int = 4, axes=PLAN_AXES, log=None) -> dict:
     ({"block": 1}) unless one of them beats it."""
     best = {name: int(plan.info(name)) for name, _ in axes}  # the library's default shape first
     block_rate = 0.0
-    try:
-        block = plan.info("block") > 0
-    except (KeyError, FDTD2DError):
-        block = False
+    block = _block_form(plan)
     if block:
         _plan_trial(plan, launches)
         block_rate = _plan_trial(plan, launches)
@@ -208,9 +232,10 @@ def tune_plan(plan, launches: int = 4, axes=PLAN_AXES, log=None) -> dict:
 
 def plan_shape(plan, key: str, cus: int, cache: "ShapeCache | None", tune: bool = False, log=None) -> dict:
     """Sets the plan's launch shape from the cache entry for `key` (kind
-    "plan"); on a miss, with tune, runs tune_plan on the plan and stores the
-    result, else leaves the library's defaults. Returns {"shape", "source",
-    "key", "trials"}."""
+    "plan") in the form the plan runs in (form_key); on a miss, with tune, runs
+    tune_plan on the plan and stores the result, else leaves the library's
+    defaults. Returns {"shape", "source", "key", "trials"}."""
+    key = form_key(key, _block_form(plan))
     if cache is not None:
         shape, src = cache.lookup("plan", key, cus)
         if shape is not None:

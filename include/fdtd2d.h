@@ -444,7 +444,9 @@ int fdtd2d_plan_kernel_time(fdtd2d_plan *plan, int cls, double *avg_ms, int *cou
  * "budget_bytes" (before any shot: carve shots from one arena of that size
  * and refuse shots that do not fit, FDTD2D_ENOMEM).
  * Info (fdtd2d_pool_get_info): the options ("block": 1 when the next launch
- * of the shots in the pool runs in that form), "bytes_in_use", "largest_free",
+ * of the shots in the pool runs in that form), "block_cells_density" and
+ * "block_cells_table" (cells up to which it does by itself), "bytes_in_use",
+ * "largest_free",
  * "shots", "running", "launches", "cell_updates", "graph_replays",
  * "eager_launches", "tail_launches", "cus", and host-side counters:
  * "rebuilds" / "captures" (main tile lists rebuilt, graphs captured),

@@ -9,6 +9,7 @@ import pytest
 
 import fdtd2d_amd as F
 from fdtd2d_amd import batch
+from fdtd2d_amd.tuning import ShapeCache, mix_key
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +72,20 @@ def test_autotune_tries_the_block_form_only_where_it_runs(gpu_device, n, shots, 
         assert any("block" in shape for shape, _ in rec["trials"]) == block
         assert rec["rate"] > 0
         assert pool.info("block") == (1 if "block" in rec["shape"] else 0)
+
+
+def test_run_pool_of_few_shots_keeps_the_block_form(gpu_device, tmp_path):
+    """Five shots whose size shares are those of a shipped streaming shape,
+    tuned on 344 million cells: that shape is not theirs."""
+    shots = [F.Setup.box(n, n, 4, 240, 1e-3) for n in (1024, 2000, 2000, 2000, 2000)]
+    cache = ShapeCache(tmp_path / "shapes.json")
+    key = mix_key(batch.shot_sizes(shots))
+    assert cache.lookup("pool", key, 256, nearest=True)[0] is not None
+    pool, ids, st = batch.run_pool(shots, gpu_device, cache=cache)
+    with pool:
+        print(st["tuned"]["key"], st["tuned"]["shape"], flush=True)
+        assert st["tuned"]["source"] == "trials" and st["tuned"]["shape"].get("block") == 1
+        assert all(pool.state(i)[2] for i in ids)
+    pool, ids, st = batch.run_pool(shots, gpu_device, cache=cache)
+    with pool:
+        assert st["tuned"]["trials"] == [] and st["tuned"]["shape"].get("block") == 1
