@@ -224,7 +224,7 @@ def tune_plan(plan, launches: int = 4, axes=PLAN_AXES, log=None) -> dict:
             if rate > best_rate:
                 best_rate, best[name] = rate, v
         plan.set_option(name, best[name])
-    if block_rate > best_rate:
+    if block and block_rate >= best_rate:  # (equal: no steps left to measure either)
         plan.set_option("block", 1)
         return {"shape": {"block": 1}, "rate": block_rate, "trials": trials + [({"block": 1}, block_rate)]}
     return {"shape": best, "rate": best_rate, "trials": trials}

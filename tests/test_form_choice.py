@@ -155,3 +155,31 @@ def test_choose_shape_keeps_the_forms_apart(tmp_path, monkeypatch, gain):
     assert hit["trials"] == [] and hit["shape"] == rec["shape"] and again.info("block") == 0
     again = FakePool()
     assert batch.choose_shape(again, "m1|11:10", c)["trials"] == [] and again.info("block") == (1 if gain > 0 else 0)
+
+
+def _plan_trial(block_rate, stream_rate):
+    def trial(plan, launches):
+        if plan.n + 8 * launches > plan.nsteps:
+            return 0.0
+        plan.run(8 * launches)
+        return block_rate if plan.info("block") else stream_rate
+
+    return trial
+
+
+@pytest.mark.parametrize("block_rate,stream_rate,nsteps,block", [
+    (5e11, 1e11, 4000, 1),  # the block form wins
+    (1e11, 5e11, 4000, 0),  # a streaming shape does
+    (5e11, 1e11, 70, 1),    # no steps left for a streaming trial
+    (5e11, 1e11, 20, 1),    # nor for any: nothing measured, nothing changed
+])
+def test_tune_plan_leaves_the_block_form_only_for_a_better_shape(monkeypatch, block_rate, stream_rate, nsteps, block):
+    monkeypatch.setattr(tuning, "_plan_trial", _plan_trial(block_rate, stream_rate))
+    plan = FakePlan(block=1, nsteps=nsteps)
+    rec = tuning.tune_plan(plan)
+    assert plan.info("block") == block and ("block" in rec["shape"]) == bool(block)
+    assert rec["rate"] == (0.0 if nsteps < 32 else max(block_rate, stream_rate))
+    assert plan.n <= nsteps
+    # a plan in the streaming form stays there
+    plan = FakePlan(block=0, nsteps=nsteps)
+    assert "block" not in tuning.tune_plan(plan)["shape"] and plan.info("block") == 0
