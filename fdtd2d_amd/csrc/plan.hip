@@ -387,12 +387,8 @@ Tiling make_tiling(int nx, int ny, int P, int T, int C, int band, int band_cpml,
     if (!m || !m->ne_run_off) return false;
     int jl0, jl1, cs, ce;
     window(w.x, w.y, w.z, jl0, jl1, cs, ce);
-    for (int r = jl0; r < jl1; ++r) {
-      bool in = false;
-      for (int q = m->ne_run_off[r]; q < m->ne_run_off[r + 1] && !in; ++q)
-        in = m->ne_runs[q].x <= cs && m->ne_runs[q].y >= ce;
-      if (!in) return false;
-    }
+    for (int r = jl0; r < jl1; ++r)
+      if (!run_covers(m->ne_runs, m->ne_run_off[r], m->ne_run_off[r + 1], cs, ce)) return false;
     return true;
   };
   // Order by column group of 4 tiles, then first row, then tile: the 4 waves
@@ -463,11 +459,7 @@ bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMa
       bool jz = !(m && m->ne_lo), full = m && m->ne_run_off && j0 < je;
       for (int r = j0; r < je; ++r) {
         if (!jz) jz = span_hits(m->ne_lo, m->ne_hi, r, t.cs, c1) || span_hits(m->jz_lo, m->jz_hi, r, t.cs, c1);
-        if (!full) continue;
-        bool in = false;
-        for (int q = m->ne_run_off[r]; q < m->ne_run_off[r + 1] && !in; ++q)
-          in = m->ne_runs[q].x <= t.cs && m->ne_runs[q].y >= c1;
-        full = in;
+        full = full && run_covers(m->ne_runs, m->ne_run_off[r], m->ne_run_off[r + 1], t.cs, c1);
       }
       t.y_waves |= !plain_rows(rb - 1, rb + R) << w;
       t.e_waves |= ev << w;

@@ -34,6 +34,22 @@ inline void scan_runs(int n, Positive positive, Emit emit) {
   if (run >= 0) emit(run, n);
 }
 
+// Whether one of a row's runs r[first] .. r[end - 1], in order as scan_runs
+// emits them, covers [c0, c1): the last that starts at or before c0 does, or
+// none. (Tiles ask this of every row they load, and a medium of single plasma
+// cells has thousands of runs a row: looked through one by one, the tiles of a
+// 3800^2 checkerboard took 33 of 73 ms of plan creation.)
+template <class Run>
+inline bool run_covers(const Run *r, int first, int end, int c0, int c1) {
+  int lo = first, hi = end;  // runs before lo start at or before c0, runs from hi on after it
+  while (lo < hi) {
+    const int mid = lo + (hi - lo) / 2;
+    if (r[mid].x <= c0) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo > first && r[lo - 1].y >= c1;
+}
+
 }  // namespace fdtd2d
 
 #endif
