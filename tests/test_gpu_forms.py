@@ -10,6 +10,9 @@ import pytest
 import fdtd2d_amd as F
 from fdtd2d_amd import batch
 from fdtd2d_amd.tuning import ShapeCache, mix_key
+from oracle.oracle import Oracle
+
+from helpers import all_state, random_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -89,3 +92,80 @@ def test_run_pool_of_few_shots_keeps_the_block_form(gpu_device, tmp_path):
     pool, ids, st = batch.run_pool(shots, gpu_device, cache=cache)
     with pool:
         assert st["tuned"]["trials"] == [] and st["tuned"]["shape"].get("block") == 1
+
+
+@pytest.mark.parametrize("table,below,above", [(False, 3872, 3874), (True, 4898, 4900)])
+def test_plan_limits(gpu_device, table, below, above):
+    """Grids just below and above 15 million cells (density), 24 million (table)."""
+    for n, block in ((below, 1), (above, 0)):
+        with F.Plan(_problem(n, n, table, nsteps=8), gpu_device) as plan:
+            assert plan.info("block") == block
+            plan.run(8)
+            plan.sync()
+
+
+def _same(got, want, label):
+    """Equal bits, where neither is a NaN; those in the same places."""
+    for k in want:
+        g, w = (np.asarray(v, np.float32) for v in (got[k], want[k]))
+        assert np.array_equal(np.isnan(g), np.isnan(w)), f"{label}: {k}: NaN elsewhere"
+        ok = ~np.isnan(w)
+        assert np.array_equal(g[ok].view(np.uint32), w[ok].view(np.uint32)), f"{label}: {k} differs"
+
+
+@pytest.mark.parametrize("table", [False, True])
+def test_infinities_and_nan_cross_tile_edges(gpu_device, table):
+    """Infinities, a NaN and the largest values put beside the edges of tiles
+    and of their waves' rows, in plasma and out of it: they spread one cell a
+    step and no further, in every shape of either form."""
+    p = random_problem(np.random.default_rng(31 + table), nx=420, ny=230, npml=8, nsteps=21, table=table)
+    ez = np.zeros((p.ny, p.nx), np.float32)
+    # a first column piece ends at 56; a further one stores 48, 112 columns wide
+    # ones follow; rows of a wave end every 2, 3, 4 or 6, those of a tile at 16 .. 64
+    for j, i, v in ((39, 55, np.inf), (40, 168, -np.inf), (103, 104, np.nan), (119, 56, 3e38), (64, 167, -3e38),
+                    (160, 279, np.inf), (199, 391, np.nan)):
+        ez[j, i] = v
+    ref = Oracle(p, 32, threads=4)
+    ref.write_field(F.EZ, ez)
+    ref.run(p.nsteps)
+    want = all_state(ref, p.npml)
+    wild = ~np.isfinite(want["ez"])
+    assert 1000 < wild.sum() < 0.5 * wild.size
+    for shape in (0, 3, 4) if table else (0, 2, 3, 4):
+        with F.Plan(p, gpu_device) as plan:
+            plan.set_option("block", shape)
+            assert plan.info("block") == (shape > 0)
+            plan.write_field(F.EZ, ez)
+            for n in (8, 5, 8):
+                plan.run(n)
+            _same(all_state(plan, p.npml), want, f"shape {shape}")
+
+
+def test_block_form_with_slicing(gpu_device):
+    """The block form switched on in a time-sliced pool: the two alternating
+    shot sets, tails at turns, slicing switched off on the way."""
+    rng = np.random.default_rng(61)
+    sizes = [(100, 90), (310, 320), (140, 77), (301, 330), (90, 130)]
+    probs = [random_problem(rng, nx=nx, ny=ny, npml=int(rng.choice([0, 5, 12])), nsteps=int(rng.integers(40, 75)),
+                            table=False) for nx, ny in sizes]
+    with F.Pool(gpu_device, graph_chunk=4, slice_cells=250 * 250, slice_every=3) as pool:
+        ids = [pool.add(p) for p in probs[:4]]
+        assert pool.info("block") == 0
+        pool.set_option("block", 1)
+        assert pool.info("block") == 1
+        pool.step(5)
+        assert pool.info("block") == 1 and pool.info("list_switches") > 0
+        ids.append(pool.add(probs[4]))
+        pool.step(6)
+        pool.set_option("slice_cells", 0)
+        while pool.info("running") > 0:
+            pool.step(4)
+        pool.sync()
+        for sid, p in zip(ids, probs):
+            ref = Oracle(p, 32, threads=4)
+            ref.run(p.nsteps)
+            det, comp = pool.read_detectors(sid)
+            rdet, rcomp = ref.read_detectors()
+            got = {"det": det, "comp": comp, **{w: pool.read_field(sid, w) for w in (F.EZ, F.HX, F.HY, F.JZ)}}
+            want = {"det": rdet, "comp": rcomp, **{w: ref.read_field(w) for w in (F.EZ, F.HX, F.HY, F.JZ)}}
+            _same(got, want, f"shot {sid} {p.nx}x{p.ny} steps {p.nsteps}")
