@@ -809,17 +809,25 @@ static void plasma_runs(const fdtd2d_problem *p, fdtd2d_plan *pl) {
 static float *pack_buffer(fdtd2d_plan *pl, size_t row) {
   if (pl->static_lists) return nullptr;
   PackBuffer &b = *pl->pack;
-  if (!b.d) {
-    // a plan's own: no more than its largest field
-    const size_t need = pl->pooled ? kPackBytes : std::min(kPackBytes, static_cast<size_t>(pl->L.ny) * pl->L.nx * 4);
-    if (hipMalloc(reinterpret_cast<void **>(&b.d), need) != hipSuccess) {
+  const size_t field = std::min(kPackBytes, static_cast<size_t>(pl->L.ny) * pl->L.nx * 4);
+  if (b.bytes < field) {
+    const size_t want = pl->pooled ? std::min(kPackBytes, std::max({field, 2 * b.bytes, kPackLeast})) : field;
+    float *d = nullptr;
+    if (hipMalloc(reinterpret_cast<void **>(&d), want) == hipSuccess) {
+      if (b.d) b.outgrown.push_back(b.d);
+      b.d = d;
+      b.bytes = want;
+    } else {
       (void)hipGetLastError();
-      b.d = nullptr;
-      return nullptr;
     }
-    b.bytes = need;
   }
   return row <= b.bytes ? b.d : nullptr;
+}
+
+void free_pack(PackBuffer &b) {
+  if (b.d) hipFree(b.d);
+  for (float *d : b.outgrown) hipFree(d);
+  b = PackBuffer();
 }
 
 // rows x cols floats between packed (row length cols) and one or two pitched
@@ -1761,7 +1769,7 @@ int fdtd2d_plan_destroy(fdtd2d_plan *pl) {
   } else if (pl->wg_buf && !pl->static_lists) {
     hipFree(pl->wg_buf);
   }
-  if (pl->own_pack.d) hipFree(pl->own_pack.d);
+  free_pack(pl->own_pack);
   if (pl->base && pl->owns_base) hipFree(pl->base);
   if (pl->aux) hipStreamDestroy(pl->aux);
   if (pl->own_stream) hipStreamDestroy(pl->own_stream);

@@ -108,17 +108,20 @@ BlockShape block_shape_for(double cells, int medium_kind);
 bool make_blocks(int nx, int ny, int P, int T, const BlockShape &s, const TileMasks *m,
                  std::vector<fdtd2d::BlockTile> &out);
 
-// Device rows packed for a copy to or from the host (copy_rows), allocated at
-// the first copy that needs it, kept and freed by its owner: a plan, or a pool
-// for all of its shots.
-constexpr size_t kPackBytes = size_t{16} << 20;
+// Device rows packed for a copy to or from the host (copy_rows): allocated at
+// the first copy that needs it, kept by its owner, a plan or a pool for all of
+// its shots. A pool's grows with the shots it reads, up to kPackBytes; the
+// smaller ones before it (less than twice that in all) are freed with it only.
+constexpr size_t kPackBytes = size_t{16} << 20, kPackLeast = size_t{1} << 20;
 struct PackBuffer {
   float *d = nullptr;
   size_t bytes = 0;
+  std::vector<float *> outgrown;
 };
 
 Layout make_layout(const fdtd2d_problem *p, size_t n_events);
 int hip_fail(hipError_t e, const char *what);
+void free_pack(PackBuffer &b);
 
 }  // namespace detail
 }  // namespace fdtd2d

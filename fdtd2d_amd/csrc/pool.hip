@@ -1088,7 +1088,7 @@ int fdtd2d_pool_destroy(fdtd2d_pool *pp) {
   if (pp->d_q) hipFree(pp->d_q);
   if (pp->d_qt) hipFree(pp->d_qt);
   if (pp->arena.base) hipFree(pp->arena.base);
-  if (pp->pack.d) hipFree(pp->pack.d);
+  free_pack(pp->pack);
   if (pp->ev_fork) hipEventDestroy(pp->ev_fork);
   if (pp->ev_join) hipEventDestroy(pp->ev_join);
   if (pp->aux) hipStreamDestroy(pp->aux);

@@ -22,9 +22,9 @@ def _bits(a):
 
 
 def _add_long(pool):
-    """A 4000^2 shot: its 2000 launches take about 0.5 s on the device and a
+    """A 4000^2 shot: its 5000 launches take about 0.6 s on the device and a
     tenth of that to issue."""
-    return pool.add(F.Setup.box(4000, 4000, 12, 16000, 1e-3))
+    return pool.add(F.Setup.box(4000, 4000, 12, 40000, 1e-3))
 
 
 def test_finished_shot_is_read_while_others_run(gpu_device):
@@ -38,7 +38,7 @@ def test_finished_shot_is_read_while_others_run(gpu_device):
         sid = pool.add(p)
         pool.step(8)
         pool.sync()
-        pool.step(2000)
+        pool.step(5000)
         got = [pool.read_field(sid, w) for w in FIELDS]
         done = pool.state(big)
         print(f"4000^2 shot beside it: {done}", flush=True)
@@ -59,7 +59,7 @@ def test_plan_is_read_and_written_while_a_pool_runs(gpu_device):
         big = _add_long(pool)
         pool.step(8)
         pool.sync()
-        pool.step(2000)
+        pool.step(5000)
         got = {w: plan.read_field(w) for w in FIELDS}
         psi = {w: plan.read_psi(w) for w in (F.PSI_HYX, F.PSI_EZX, F.PSI_HXY, F.PSI_EZY)}
         plan.write_field(F.EZ, got[F.EZ])
@@ -85,3 +85,22 @@ def test_rows_beyond_the_packing_buffer(gpu_device, nx, ny):
             v = rng.standard_normal(plan.read_field(which).shape).astype(np.float32)
             plan.write_field(which, v)
             assert np.array_equal(_bits(plan.read_field(which)), _bits(v)), which
+
+
+def test_pool_buffer_grows_with_the_shots_read(gpu_device):
+    """Shots of 0.03, 0.24, 2.4 and 17 MB a field (the packing buffer's least
+    and most size between them), read in that order and back."""
+    rng = np.random.default_rng(43)
+    probs = [random_problem(rng, nx=nx, ny=ny, npml=5, nsteps=8, table=False)
+             for nx, ny in ((90, 70), (301, 203), (777, 803), (2049, 2101))]
+    want = []
+    for p in probs:
+        ref = Oracle(p, 32, threads=8)
+        ref.run(p.nsteps)
+        want.append({w: ref.read_field(w) for w in FIELDS})
+    with F.Pool(gpu_device) as pool:
+        ids = [pool.add(p) for p in probs]
+        pool.step(1)
+        for k in (0, 1, 2, 3, 2, 1, 0):
+            for w in FIELDS:
+                assert np.array_equal(_bits(pool.read_field(ids[k], w)), _bits(want[k][w])), (k, w)
