@@ -44,7 +44,8 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 // The step loop's barrier. The wait for the wave's own LDS writes is spelled
 // out: the compiler (ROCm 7.2) dropped the one that the barrier's release
 // fence stands for from loops whose header holds the barrier, and a wave then
-// read a neighbour's row before it had arrived (one launch in thousands).
+// read a neighbour's row before it had arrived (a pool of eight small table
+// shots: one run of 75 launches in ten had a wrong row).
 __device__ __forceinline__ void step_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();

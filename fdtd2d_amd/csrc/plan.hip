@@ -1247,8 +1247,9 @@ int fdtd2d::detail::create_plan(const fdtd2d_problem *p, int device, bool pooled
     u_hy = p->den_hy[jm];
     u_ey = p->den_ey[jm];
     auto same = [](float x, float y) { return std::memcmp(&x, &y, 4) == 0; };
-    // RC probe columns and the processing line's row are special too: only
-    // general CPML-class tiles capture them
+    // RC probe columns and the processing line's row are special too: of the
+    // streaming form's tiles only general CPML-class ones capture them, of the
+    // block form's those marked for it
     std::vector<char> probe(nx, 0);
     for (int e = 0; e < p->nrc; ++e) probe[p->rc_i[e]] = probe[p->rc_imax[e]] = 1;
     pl->scol_pref.assign(nx + 1, 0);

@@ -306,7 +306,10 @@ int fdtd2d_plan_create(const fdtd2d_problem *p, int device, fdtd2d_plan **out);
  * fdtd2d_plan_set_option), and since every such plan on a device would share
  * that array, only one may exist per device at a time (FDTD2D_ESTATE);
  * plans of fdtd2d_plan_create are unaffected. Everything else (run, read,
- * write, options, destroy, which frees nothing) works as for any plan. */
+ * write, options, destroy, which frees nothing) works as for any plan; fields
+ * and psi strips whose rows are not contiguous on the device (widths that are
+ * no multiple of 64, all of Hy, the x strips) cross a row at a time, 7-10 us
+ * each, since a plan that allocates nothing has no buffer to pack them in. */
 int fdtd2d_plan_create_in(const fdtd2d_problem *p, int device, void *mem, size_t bytes, void *stream,
                           fdtd2d_plan **out);
 /* Work on `stream` (a hipStream_t; NULL = the plan's own stream). */
@@ -353,6 +356,10 @@ int fdtd2d_steps_done(const fdtd2d_plan *plan, int *n);
 /* Traces: det [(nsteps+1)*ndet], comp [3][(nsteps+1)*ncomp] as Ez, Hx, Hy. */
 int fdtd2d_read_detectors(fdtd2d_plan *plan, float *det, size_t det_count, float *comp,
                           size_t comp_count);
+/* Fields. Rows that are not contiguous on the device pass a packing buffer of
+ * at most 16 MiB that the plan (a pool for its shots: up to 32 MiB with the
+ * ones it outgrew) allocates at the first such call and keeps, outside "bytes"
+ * and "budget_bytes". */
 int fdtd2d_read_field(fdtd2d_plan *plan, int which, float *out, size_t count);
 int fdtd2d_write_field(fdtd2d_plan *plan, int which, const float *in, size_t count);
 /* psi strips, reference layouts (F/kernel.cu:1172-1214): HXY [2][npml-1][nx],
