@@ -42,11 +42,12 @@ inline void scan_runs(int n, Positive positive, Emit emit) {
 template <class Run>
 inline bool run_covers(const Run *r, int first, int end, int c0, int c1) {
   int lo = first, hi = end;  // runs before lo start at or before c0, runs from hi on after it
-  while (lo < hi) {
+  while (hi - lo > 4) {
     const int mid = lo + (hi - lo) / 2;
     if (r[mid].x <= c0) lo = mid + 1;
     else hi = mid;
   }
+  while (lo < hi && r[lo].x <= c0) ++lo;  // (most rows hold one run)
   return lo > first && r[lo - 1].y >= c1;
 }
 
